@@ -135,8 +135,12 @@ __global__ void __launch_bounds__(256) awq_prescale_split_kernel(
 
 __global__ void __launch_bounds__(256) awq_glu_kernel(
     const uint16_t* __restrict__ gu, const int32_t* __restrict__ offsets, int E, int I,
-    const uint16_t* __restrict__ s_dn, int act, float alpha, float limit, uint16_t* __restrict__ h) {
+    const uint16_t* __restrict__ s_dn, int act, float alpha, float limit, uint16_t* __restrict__ h,
+    int cls, int split_rows) {
   const int64_t m = blockIdx.x;
+  int e = 0;
+  if (s_dn || cls != kAllExperts) e = expert_of_row(offsets, E, m);
+  if (cls != kAllExperts && (offsets[e + 1] - offsets[e] > split_rows) != (cls == kHotExperts)) return;
   const u32x4* g4 = reinterpret_cast<const u32x4*>(gu + m * 2 * I);
   const u32x4* u4 = g4 + I / 8;
   u32x4* o4 = reinterpret_cast<u32x4*>(h + m * I);
@@ -152,7 +156,6 @@ __global__ void __launch_bounds__(256) awq_glu_kernel(
     }
     return;
   }
-  const int e = expert_of_row(offsets, E, m);
   const u32x4* s4 = reinterpret_cast<const u32x4*>(s_dn + static_cast<int64_t>(e) * I);
   for (int i = threadIdx.x; i < I / 8; i += 256) {
     const u32x4 g = g4[i], u = u4[i], s = s4[i];
@@ -202,12 +205,12 @@ int launch_awq_prescale_split(const uint16_t* x, const int32_t* sorted, const in
 
 int launch_awq_glu(const uint16_t* gu, const int32_t* offsets, int E, int64_t mc, int I,
                    const uint16_t* s_dn, int act, float alpha, float limit, uint16_t* h,
-                   hipStream_t stream) {
+                   hipStream_t stream, int cls, int split_rows) {
   if (mc <= 0) return 0;
   if (I <= 0 || I % 8) return fail("awq glu: I % 8 == 0 required");
   if (mc > 0x7fffffff) return fail("awq glu: too many rows");
   awq_glu_kernel<<<static_cast<unsigned>(mc), 256, 0, stream>>>(gu, offsets, E, I, s_dn, act, alpha,
-                                                                 limit, h);
+                                                                 limit, h, cls, split_rows);
   return check_launch("awq glu");
 }
 

@@ -293,15 +293,15 @@ int validate_routing(int N, int H, int E, int k, int scoring, int n_group, int t
 //    than the shared expert's bytes);
 //  * in the hybrid regime, the cold experts' grouped matmuls (small kernel, bound by HBM)
 //    beside the hot experts' (large kernel, bound by MFMA).
-// A fork event records the caller's stream at entry, `perm` publishes the permute to the
-// auxiliary stream, `cold` returns the cold gate_up (h complete), `hready` publishes the fp16
-// copy of h, and the caller's stream waits on `join` right before the combine. The mutex is held
+// A fork event records the caller's stream at entry, `xready` returns the fp16 copy of x, `perm`
+// publishes the permute to the auxiliary stream, and the caller's stream waits on `join` right
+// before the combine: the cold experts' gate_up and down and the hot experts' are two chains over
+// disjoint rows of h and d, with no event between them (each wait costs the stream about 6 us). The mutex is held
 // from the fork record until the join wait is enqueued, so concurrent calls on different streams
 // cannot exchange the events.
 struct AuxStream {
   hipStream_t s = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr, perm = nullptr, cold = nullptr, hready = nullptr,
-             xready = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr, perm = nullptr, xready = nullptr;
 };
 static std::mutex g_aux_mu;
 constexpr int64_t kFuseSharedMaxTokens = 64;
@@ -354,8 +354,6 @@ static int aux_stream(hipStream_t caller, AuxStream** out) {
     if (err == hipSuccess) err = hipEventCreateWithFlags(&a.fork, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&a.join, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&a.perm, hipEventDisableTiming);
-    if (err == hipSuccess) err = hipEventCreateWithFlags(&a.cold, hipEventDisableTiming);
-    if (err == hipSuccess) err = hipEventCreateWithFlags(&a.hready, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&a.xready, hipEventDisableTiming);
     if (cur != dev) (void)hipSetDevice(cur);
     if (err != hipSuccess) {
@@ -369,16 +367,39 @@ static int aux_stream(hipStream_t caller, AuxStream** out) {
 
 // Large-M tiles pay off once a batch gives experts tens of rows; they also need the output
 // widths (hidden for the down projection) to be multiples of the 256-row tile.
-static int dense_regime(const qmoe_config_t& c, int64_t N) {
-  return (N > 256 && c.hidden % 256 == 0) ? QMOE_REGIME_LARGE : QMOE_REGIME_SMALL;
+static bool large_ok(const qmoe_config_t& c, int64_t N) { return N > 256 && c.hidden % 256 == 0; }
+
+// Regime of a dense product (router, shared expert) of `rows` weight rows over K: the decode kernel
+// up to 256 tokens (outputs that do not depend on the batch), above that qmm_dense_kernel's 64 x 64
+// tiles, which fill the chip with small products; the large kernel's 128 x 256 tiles from the sizes
+// where they fill it too and their fewer bytes from L2 win. Whole layers, us, 64 x 64 against 128 x
+// 256 tiles: c1 391 tokens 168 / 249, c2 512 (AWQ) 887 / 946, c2 1000 960 / 991, c3 300 1285 / 1356;
+// c2 2000 1200 / 1174, c2 4096 1901 / 1850.
+constexpr double kDenseLargeMacs = 4e9;
+constexpr int64_t kDenseLargeTokens = 1536;
+static int dense_regime(const qmoe_config_t& c, int64_t N, int64_t rows, int64_t K) {
+  if (N <= 256) return QMOE_REGIME_SMALL;
+  return large_ok(c, N) && N > kDenseLargeTokens && static_cast<double>(N) * rows * K >= kDenseLargeMacs
+             ? QMOE_REGIME_LARGE : kRegimeDense;
+}
+static int shared_gu_regime(const qmoe_config_t& c, int64_t N) {
+  return dense_regime(c, N, 2 * static_cast<int64_t>(c.shared_inter), c.hidden);
+}
+static int shared_dn_regime(const qmoe_config_t& c, int64_t N) {
+  return dense_regime(c, N, c.hidden, c.shared_inter);
 }
 
-// Whether an int8 shared expert is expanded to bf16 for this call: the large-M kernel stages
-// bf16 (or int4) weights only, and above the decode sizes the expansion (half the bf16 bytes
-// read, all of them written once) is small beside the block.
-static bool shared_expands(const qmoe_config_t& c, int64_t N) {
-  return c.shared_inter > 0 && c.shared_format == QMOE_FMT_INT8_G64 &&
-         dense_regime(c, N) == QMOE_REGIME_LARGE;
+// Whether a projection of an int8 shared expert is expanded to bf16 for this call: the large-M
+// kernel stages bf16 (or int4) weights only, and at its sizes the expansion (half the bf16 bytes
+// read, all of them written once) is small beside the product.
+static bool shared_int8(const qmoe_config_t& c) {
+  return c.shared_inter > 0 && c.shared_format == QMOE_FMT_INT8_G64;
+}
+static bool expand_gu(const qmoe_config_t& c, int64_t N) {
+  return shared_int8(c) && shared_gu_regime(c, N) == QMOE_REGIME_LARGE;
+}
+static bool expand_dn(const qmoe_config_t& c, int64_t N) {
+  return shared_int8(c) && shared_dn_regime(c, N) == QMOE_REGIME_LARGE;
 }
 
 // ------------------------------------------------------------------ forward workspace layout
@@ -423,7 +444,7 @@ static WsLayout ws_layout(const qmoe_config_t& c, int64_t N) {
   L.sh_out = take(static_cast<size_t>(N) * (c.shared_inter > 0 ? c.hidden : 0) * 2);
   // int8 shared expert above the decode sizes: its weights expanded to tiled bf16 for the
   // large-M kernel (gate|up [2 Is, H] then down [H, Is])
-  L.sh_w16 = take(shared_expands(c, N) ? static_cast<size_t>(3) * c.shared_inter * c.hidden * 2 : 0);
+  L.sh_w16 = take((expand_gu(c, N) || expand_dn(c, N)) ? static_cast<size_t>(3) * c.shared_inter * c.hidden * 2 : 0);
   // fp16 per-row-scaled activation copies for the large-M int4 regime (AWQ: of the gate's and
   // the up projection's prescaled rows, [2][mc])
   const int64_t x16_rows = c.awq ? 2 * mc : N;
@@ -638,7 +659,7 @@ extern "C" int qmoe_set_route_tail(int on) {
 static int pick_regime(const qmoe_config_t& c, int64_t N) {
   if (c.regime != QMOE_REGIME_AUTO) return c.regime;
   if (c.awq && !awq_large_ok(c)) return QMOE_REGIME_SMALL;
-  return dense_regime(c, N);
+  return large_ok(c, N) ? QMOE_REGIME_LARGE : QMOE_REGIME_SMALL;
 }
 
 // The block on x; with resid, the combine adds the decoder layer's residual row.
@@ -712,23 +733,23 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
   const int n = static_cast<int>(N);
   const int64_t mc = N * c.top_k;
   const int regime = pick_regime(c, N);
-  // Large-M regime = hybrid: experts with more than kHybridSplitRows rows run on the large
-  // kernel (128-row tiles), the rest on the small kernel (16-row tiles). A handful of rows
-  // cannot amortise a 128-row tile's weight dequant; under skewed routing most experts are
-  // that small while a few carry thousands of rows.
+  // Large-M regime = hybrid: experts with more than `split` rows run on the large kernel (128-row
+  // tiles), the rest on the small kernel (16-row tiles). A handful of rows cannot amortise a
+  // 128-row tile's weight dequant; under skewed routing most experts are that small while a few
+  // carry thousands of rows.
   const bool hybrid = (regime == QMOE_REGIME_LARGE);
+  const int split = hybrid_split_rows(mc, c.n_experts);
   int32_t* tile_map_big = reinterpret_cast<int32_t*>(base + L.tile_map_big);
   const int64_t bound_small = mtile_upper_bound(mc, c.n_experts, kSmallMTile);
   const int64_t cold_bound =
       std::min<int64_t>(bound_small, static_cast<int64_t>(c.n_experts) *
-                                         ((kHybridSplitRows + kSmallMTile - 1) / kSmallMTile));
+                                         ((split + kSmallMTile - 1) / kSmallMTile));
   const int64_t hot_bound = (mc + kLargeMTile - 1) / kLargeMTile +
-                            std::min<int64_t>(c.n_experts, mc / (kHybridSplitRows + 1));
+                            std::min<int64_t>(c.n_experts, mc / (split + 1));
   const int gfmt = kernel_fmt(c.expert_format), dfmt = kernel_fmt(c.down_format);
   const int has_sg = (c.shared_inter > 0 && c.shared_gated) ? 1 : 0;
 
-  const int sreg = dense_regime(c, N);
-  const bool decode = (sreg == QMOE_REGIME_SMALL);
+  const int reg_gu = shared_gu_regime(c, N), reg_dn = shared_dn_regime(c, N);
   // Small decode batches: the shared expert rides in the neighbouring launches, its gate_up with
   // the router logits and its down projection in the combine, so no launch or stream event of
   // its own. Otherwise the shared expert and, in the hybrid regime, the cold experts' grouped
@@ -736,14 +757,15 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
   const bool shared = c.shared_inter > 0;
   // (the fused launches give bit-identical results; above kFuseSharedMaxTokens the shared
   // expert's re-read weights cost more than the auxiliary stream's join)
-  const bool fuse = decode && shared && N <= kFuseSharedMaxTokens;
+  const bool fuse = shared && N <= kFuseSharedMaxTokens;
   const bool fuse_gu = fuse && c.router_format == QMOE_ROUTER_BF16_TILED;
   // the block's input rows: x itself, or its RMSNorm (made inside the router launch when that is
   // the fused pair, else by a launch of its own ahead of everything)
   const uint16_t* resid = norm_w ? x_in : nullptr;
   const uint16_t* x = norm_w ? xn : x_in;
   // (the router launch normalises the rows when its shape allows, pair_norm_fusable)
-  const bool fuse_norm = norm_w && fuse_gu && pair_norm_fusable(c.hidden, N);
+  // (the hybrid regime copies the normalised rows to fp16 beside the router)
+  const bool fuse_norm = norm_w && fuse_gu && !hybrid && pair_norm_fusable(c.hidden, N);
   if (norm_w && !fuse_norm) {
     rc = launch_rmsnorm(x_in, norm_w, N, c.hidden, norm_eps, xn, static_cast<hipStream_t>(stream_));
     if (rc) return rc;
@@ -789,37 +811,35 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
   }
 
   // 1. shared expert gate_up + SwiGLU -> sh_h (fused with the router below when decoding)
-  const int st = decode ? kSmallMTile : kLargeMTile;
+  auto mtiles_of = [&](int reg) {
+    const int t = (reg == QMOE_REGIME_LARGE) ? kLargeMTile : kSmallMTile;
+    return (N + t - 1) / t;
+  };
   QmmArgs sgu{};
   // the shared expert's weights as the kernels read them: int8 codes dequantized in registers,
-  // or (large regime) expanded to bf16 in the workspace first
-  int sfmt = (c.shared_format == QMOE_FMT_INT8_G64) ? FMT_INT8 : FMT_BF16;
-  const void* sh_gu_w = wts->sh_gu;
-  const void* sh_dn_w = wts->sh_dn;
-  if (shared && shared_expands(c, N)) {
-    uint16_t* w16 = reinterpret_cast<uint16_t*>(base + L.sh_w16);
-    const int64_t gu_elems = static_cast<int64_t>(2) * c.shared_inter * c.hidden;
-    rc = launch_expand_int8(reinterpret_cast<const uint32_t*>(wts->sh_gu), wts->sh_gu_sb,
-                            2 * c.shared_inter, c.hidden, w16, sstream);
-    if (!rc)
-      rc = launch_expand_int8(reinterpret_cast<const uint32_t*>(wts->sh_dn), wts->sh_dn_sb,
-                              c.hidden, c.shared_inter, w16 + gu_elems, sstream);
-    if (rc) return rc;
-    sh_gu_w = w16;
-    sh_dn_w = w16 + gu_elems;
-    sfmt = FMT_BF16;
-  }
+  // or (a projection on the large kernel) expanded to bf16 in the workspace first
+  const int sfmt = shared_int8(c) ? FMT_INT8 : FMT_BF16;
   const bool sh8 = (sfmt == FMT_INT8);
+  uint16_t* w16_gu = reinterpret_cast<uint16_t*>(base + L.sh_w16);
+  uint16_t* w16_dn = w16_gu + static_cast<int64_t>(2) * c.shared_inter * c.hidden;
+  const bool exp_gu = expand_gu(c, N), exp_dn = expand_dn(c, N);
+  const void* sh_gu_w = exp_gu ? w16_gu : wts->sh_gu;
+  const void* sh_dn_w = exp_dn ? w16_dn : wts->sh_dn;
   if (shared) {
     sgu.act = x; sgu.act_rows = N; sgu.slot_div = 1; sgu.dense_rows = N; sgu.n_experts = 1;
     sgu.K = c.hidden; sgu.n_rows = 2 * c.shared_inter; sgu.codes = sh_gu_w; sgu.out = sh_h;
-    sgu.sb = sh8 ? wts->sh_gu_sb : nullptr;
+    sgu.sb = (sh8 && !exp_gu) ? wts->sh_gu_sb : nullptr;
     sgu.ld_out = c.shared_inter;
     sgu.glu = c.act; sgu.glu_alpha = c.act_alpha; sgu.glu_limit = c.act_limit;
-    if (!fuse_gu) {
-      rc = launch_qmm(sgu, sfmt, EPI_SWIGLU, sreg, (N + st - 1) / st, sstream);
+  }
+  if (shared && !fuse_gu) {
+    if (exp_gu) {
+      rc = launch_expand_int8(reinterpret_cast<const uint32_t*>(wts->sh_gu), wts->sh_gu_sb,
+                              2 * c.shared_inter, c.hidden, w16_gu, sstream);
       if (rc) return rc;
     }
+    rc = launch_qmm(sgu, exp_gu ? FMT_BF16 : sfmt, EPI_SWIGLU, reg_gu, mtiles_of(reg_gu), sstream);
+    if (rc) return rc;
   }
   // shared down -> sh_out (fused into the combine when decoding). In the hybrid regime it is
   // enqueued on the auxiliary stream after the cold experts' launches, so it runs beside the hot
@@ -828,12 +848,18 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     QmmArgs b{};
     b.act = sh_h; b.act_rows = N; b.slot_div = 1; b.dense_rows = N; b.n_experts = 1;
     b.K = c.shared_inter; b.n_rows = c.hidden; b.codes = sh_dn_w; b.out = sh_out;
-    b.sb = sh8 ? wts->sh_dn_sb : nullptr;
+    b.sb = (sh8 && !exp_dn) ? wts->sh_dn_sb : nullptr;
     b.ld_out = c.hidden;
     return b;
   };
   auto shared_down = [&]() -> int {
-    return launch_qmm(shared_down_args(), sfmt, EPI_BF16, sreg, (N + st - 1) / st, sstream);
+    if (exp_dn) {
+      const int r = launch_expand_int8(reinterpret_cast<const uint32_t*>(wts->sh_dn), wts->sh_dn_sb,
+                                       c.hidden, c.shared_inter, w16_dn, sstream);
+      if (r) return r;
+    }
+    return launch_qmm(shared_down_args(), exp_dn ? FMT_BF16 : sfmt, EPI_BF16, reg_dn,
+                      mtiles_of(reg_dn), sstream);
   };
   // decode batches whose shared down would ride in the combine: with int8 shared weights and
   // int4 routed experts it rides in the routed gate_up's launch instead (the combine then only
@@ -877,7 +903,10 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     // are padding for the large kernel's 256-row tiles)
     const int live_rows = (c.n_experts + has_sg + 15) / 16 * 16;
     a.act = x; a.act_rows = N; a.slot_div = 1; a.dense_rows = N; a.n_experts = 1;
-    a.K = c.hidden; a.n_rows = decode ? std::min(live_rows, c.router_rows) : c.router_rows;
+    const int rreg = dense_regime(c, N, live_rows, c.hidden);
+    a.K = c.hidden;
+    a.n_rows = (rreg == QMOE_REGIME_SMALL) ? std::min(live_rows, c.router_rows)
+               : (rreg == kRegimeDense) ? (live_rows + 63) / 64 * 64 : c.router_rows;
     a.codes = wts->router_w; a.out = logits; a.ld_out = ld;
     if (fuse_norm) {   // both products read the raw rows and normalise them; the router writes xn
       a.act = x_in; a.norm_w = norm_w; a.norm_eps = norm_eps; a.norm_out = xn;
@@ -885,8 +914,8 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     }
     // (large regime: 64-token m-tiles, so the few row blocks of the router still give twice
     // as many workgroups)
-    const int rt = decode ? st : 64;
-    if (!decode) a.dense_mtile = rt;
+    const int rt = (rreg == QMOE_REGIME_LARGE) ? 64 : kSmallMTile;
+    if (rreg == QMOE_REGIME_LARGE) a.dense_mtile = rt;
     if (use_flow) {
       a.zero_words = sync;
       a.n_zero = static_cast<int>(L.sync_words / kSyncStride);
@@ -911,7 +940,7 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
       if (split) sgu.ld_out = 2 * c.shared_inter;
       rc = launch_qmm_pair_bf16(a, sgu, stream, sfmt, split);
     } else {
-      rc = launch_qmm(a, FMT_BF16, EPI_F32, sreg, (N + rt - 1) / rt, stream);
+      rc = launch_qmm(a, FMT_BF16, EPI_F32, rreg, (N + rt - 1) / rt, stream);
     }
   }
   if (rc) return rc;
@@ -954,7 +983,7 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     if (rc) return rc;
     // 4. stable permute by expert (16-row tiles; hybrid: hot experts' 128-row tiles separately)
     rc = launch_permute(idx, n, c.top_k, c.n_experts, kSmallMTile, counts, offsets, tile_off,
-                        sorted, inv, tile_map, bound_small, stream, kHybridSplitRows, kLargeMTile,
+                        sorted, inv, tile_map, bound_small, stream, split, kLargeMTile,
                         hybrid ? tile_map_big : nullptr, L.max_tiles_big);
     if (rc) return rc;
   }
@@ -964,7 +993,7 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
   if (c.awq && hybrid && c.hidden <= kAwqSplitMaxH) {
     // (hot experts' rows only as their fp16 copies, cold experts' only as bf16)
     rc = launch_awq_prescale_split(x, sorted, offsets, c.n_experts, c.top_k, mc, c.hidden,
-                                   wts->awq_gu, kHybridSplitRows, awq_xg, x16, x_sinv, stream);
+                                   wts->awq_gu, split, awq_xg, x16, x_sinv, stream);
     if (rc) return rc;
   } else if (c.awq) {
     rc = launch_awq_prescale(x, sorted, offsets, c.n_experts, c.top_k, mc, c.hidden, wts->awq_gu,
@@ -972,98 +1001,69 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     if (!rc && hybrid) rc = launch_act_to_f16(awq_xg, 2 * mc, c.hidden, x16, x_sinv, stream);
     if (rc) return rc;
   }
-  // the cold experts' tiles wait for the permute on the auxiliary stream
-  hipStream_t cstream = stream;
+  // The shorter chain takes the auxiliary stream, behind the permute: the cold experts', or the hot
+  // ones' where few experts are hot. (c1, 391 tokens: 168 us per layer, 186 with the long chain there.)
+  hipStream_t cstream = stream, hstream = stream;
   if (hybrid && aux) {
     rc = link(aux->perm, stream, aux->s, "permute to auxiliary stream");
     if (rc) return rc;
-    cstream = aux->s;
+    (few_hot(mc, c.n_experts) ? hstream : cstream) = aux->s;
   }
-  // routed grouped matmul over the permuted rows: small kernel over the (cold) 16-row tiles,
-  // large kernel over the hot experts' tiles (hybrid: the two on different streams; hot and
-  // cold experts own disjoint rows of the output)
-  auto routed = [&](QmmArgs a, int fmt, int epi, const uint16_t* act16, const float* sinv) {
-    a.tile_map = reinterpret_cast<const int4*>(tile_map);
-    int r = launch_qmm(a, fmt, epi, QMOE_REGIME_SMALL, hybrid ? cold_bound : tiles_small, cstream);
-    if (r || !hybrid) return r;
+  // routed grouped matmul over the permuted rows of one class of experts: all of them on the small
+  // kernel, or (hybrid) the cold ones there over their 16-row tiles and the hot ones on the large
+  // kernel. The two classes own disjoint rows of h and d.
+  auto routed = [&](QmmArgs a, int fmt, int epi, const uint16_t* act16, const float* sinv, ExpertClass cls) {
+    if (cls != kHotExperts) {
+      a.tile_map = reinterpret_cast<const int4*>(tile_map);
+      return launch_qmm(a, fmt, epi, QMOE_REGIME_SMALL, hybrid ? cold_bound : tiles_small, cstream);
+    }
     a.tile_map = reinterpret_cast<const int4*>(tile_map_big);
     a.act16 = act16;
     a.row_sinv = sinv;
-    return launch_qmm(a, fmt, epi, QMOE_REGIME_LARGE, hot_bound, stream);
+    return launch_qmm(a, fmt, epi, QMOE_REGIME_LARGE, hot_bound, hstream);
   };
-  if (f16_acts && aux) {   // the fp16 copy of x, made on the auxiliary stream at the fork
-    const hipError_t err = hipStreamWaitEvent(stream, aux->xready, 0);
-    if (err != hipSuccess) return fail(std::string("forward: x16 wait: ") + hipGetErrorString(err));
-  }
   // 5. routed gate_up + SwiGLU -> h (sorted order)
-  if (mixed && !has_split(*mixed)) {
-    // fused gate_up stacks by width: SwiGLU in the epilogue, straight into h
-    for (int i = 0; i < mixed->n_stacks; ++i) {
-      const qmoe_stack_t& st = mixed->stacks[i];
-      if (st.proj != QMOE_PROJ_GATE_UP) continue;
-      QmmArgs a{};
-      a.act = x; a.act_rows = N; a.slot_of = sorted; a.slot_div = c.top_k; a.n_slots = mc;
-      a.offsets = offsets; a.tile_off = tile_off; a.n_experts = c.n_experts;
-      a.K = c.hidden; a.n_rows = 2 * c.inter; a.codes = st.codes; a.sb = st.sb;
-      a.expert_map = st.expert_slot; a.out = h; a.ld_out = c.inter;
-      a.row_exp = st.row_exp;
+  auto gate_up = [&](ExpertClass cls) -> int {
+    QmmArgs a{};
+    a.n_slots = mc; a.offsets = offsets; a.tile_off = tile_off; a.n_experts = c.n_experts;
+    a.K = c.hidden;
+    if (mixed) {
+      // fused gate_up stacks by width, SwiGLU in the epilogue, straight into h; or widths per
+      // (expert, projection): gate and up by width into awq_gu, then h = bf16(glu)
+      const bool halves = has_split(*mixed);
+      uint16_t* gu = reinterpret_cast<uint16_t*>(base + L.awq_gu);
+      a.act = x; a.act_rows = N; a.slot_of = sorted; a.slot_div = c.top_k;
+      a.n_rows = halves ? c.inter : 2 * c.inter;
+      a.out = h; a.ld_out = halves ? 2 * c.inter : c.inter;
       a.glu = c.act; a.glu_alpha = c.act_alpha; a.glu_limit = c.act_limit;
-      rc = routed(a, kernel_fmt(st.format), EPI_SWIGLU, x16, x_sinv);
-      if (rc) return rc;
+      for (int i = 0; i < mixed->n_stacks; ++i) {
+        const qmoe_stack_t& st = mixed->stacks[i];
+        if (st.proj == QMOE_PROJ_DOWN) continue;
+        a.codes = st.codes; a.sb = st.sb; a.expert_map = st.expert_slot; a.row_exp = st.row_exp;
+        if (halves) a.out = gu + (st.proj == QMOE_PROJ_UP ? c.inter : 0);
+        const int r = routed(a, kernel_fmt(st.format), halves ? EPI_BF16 : EPI_SWIGLU, x16, x_sinv, cls);
+        if (r) return r;
+      }
+      if (!halves) return 0;
+      return launch_awq_glu(gu, offsets, c.n_experts, mc, c.inter, nullptr, c.act, c.act_alpha,
+                            c.act_limit, h, cls == kHotExperts ? hstream : cstream, cls, split);
     }
-    if (hybrid && aux) {   // h complete (cold rows from the auxiliary stream)
-      rc = link(aux->cold, aux->s, stream, "cold gate_up");
-      if (rc) return rc;
-    }
-  } else if (mixed) {
-    // widths per (expert, projection): gate and up by width into awq_gu, then h = bf16(glu)
-    uint16_t* gu = reinterpret_cast<uint16_t*>(base + L.awq_gu);
-    for (int i = 0; i < mixed->n_stacks; ++i) {
-      const qmoe_stack_t& st = mixed->stacks[i];
-      if (st.proj != QMOE_PROJ_GATE && st.proj != QMOE_PROJ_UP) continue;
-      QmmArgs a{};
-      a.act = x; a.act_rows = N; a.slot_of = sorted; a.slot_div = c.top_k; a.n_slots = mc;
-      a.offsets = offsets; a.tile_off = tile_off; a.n_experts = c.n_experts;
-      a.K = c.hidden; a.n_rows = c.inter; a.codes = st.codes; a.sb = st.sb;
-      a.expert_map = st.expert_slot; a.row_exp = st.row_exp;
-      a.out = gu + (st.proj == QMOE_PROJ_UP ? c.inter : 0); a.ld_out = 2 * c.inter;
-      rc = routed(a, kernel_fmt(st.format), EPI_BF16, x16, x_sinv);
-      if (rc) return rc;
-    }
-    if (hybrid && aux) {   // all of gu (cold rows from the auxiliary stream) before the glu pass
-      rc = link(aux->cold, aux->s, stream, "cold gate_up");
-      if (rc) return rc;
-    }
-    rc = launch_awq_glu(gu, offsets, c.n_experts, mc, c.inter, nullptr, c.act, c.act_alpha,
-                        c.act_limit, h, stream);
-    if (rc) return rc;
-  } else if (c.awq) {
-    // AWQ: gate and up on their own prescaled rows (one launch over all 2I rows of each expert,
-    // the up half's tiles reading the up rows) into awq_gu, then h = bf16(glu / s_dn)
-    uint16_t* gu = reinterpret_cast<uint16_t*>(base + L.awq_gu);
-    QmmArgs a{};
-    a.act = awq_xg; a.act_hi = awq_xg + mc * c.hidden; a.split_tile = c.inter / 16;
-    a.act_rows = mc; a.slot_div = 1; a.n_slots = mc;
-    a.offsets = offsets; a.tile_off = tile_off; a.n_experts = c.n_experts;
-    a.K = c.hidden; a.n_rows = 2 * c.inter; a.codes = wts->gu_codes; a.sb = wts->gu_sb;
+    a.n_rows = 2 * c.inter; a.codes = wts->gu_codes; a.sb = wts->gu_sb;
     a.row_exp = fp16_large_fmt(gfmt) ? wts->gu_rexp : nullptr;
-    a.out = gu; a.ld_out = 2 * c.inter;
-    if (hybrid) { a.act16_hi = x16 + mc * c.hidden; a.row_sinv_hi = x_sinv + mc; }
-    rc = routed(a, gfmt, EPI_BF16, x16, x_sinv);
-    if (rc) return rc;
-    if (hybrid && aux) {   // all of gu (cold rows from the auxiliary stream) before the glu pass
-      rc = link(aux->cold, aux->s, stream, "cold gate_up");
-      if (rc) return rc;
+    if (c.awq) {
+      // AWQ: gate and up on their own prescaled rows (one launch over all 2I rows of each expert,
+      // the up half's tiles reading the up rows) into awq_gu, then h = bf16(glu / s_dn)
+      uint16_t* gu = reinterpret_cast<uint16_t*>(base + L.awq_gu);
+      a.act = awq_xg; a.act_hi = awq_xg + mc * c.hidden; a.split_tile = c.inter / 16;
+      a.act_rows = mc; a.slot_div = 1;
+      a.out = gu; a.ld_out = 2 * c.inter;
+      if (hybrid) { a.act16_hi = x16 + mc * c.hidden; a.row_sinv_hi = x_sinv + mc; }
+      const int r = routed(a, gfmt, EPI_BF16, x16, x_sinv, cls);
+      if (r) return r;
+      return launch_awq_glu(gu, offsets, c.n_experts, mc, c.inter, wts->awq_dn, c.act, c.act_alpha,
+                            c.act_limit, h, cls == kHotExperts ? hstream : cstream, cls, split);
     }
-    rc = launch_awq_glu(gu, offsets, c.n_experts, mc, c.inter, wts->awq_dn, c.act, c.act_alpha,
-                        c.act_limit, h, stream);
-    if (rc) return rc;
-  } else {
-    QmmArgs a{};
-    a.act = x; a.act_rows = N; a.slot_of = sorted; a.slot_div = c.top_k; a.n_slots = mc;
-    a.offsets = offsets; a.tile_off = tile_off; a.n_experts = c.n_experts;
-    a.K = c.hidden; a.n_rows = 2 * c.inter; a.codes = wts->gu_codes; a.sb = wts->gu_sb;
-    a.row_exp = fp16_large_fmt(gfmt) ? wts->gu_rexp : nullptr;
+    a.act = x; a.act_rows = N; a.slot_of = sorted; a.slot_div = c.top_k;
     a.out = h; a.ld_out = c.inter;
     a.glu = c.act; a.glu_alpha = c.act_alpha; a.glu_limit = c.act_limit;
     // (the fused tail below computes the shared down itself)
@@ -1074,70 +1074,79 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
       const QmmArgs sdn = shared_down_args();
       // (the fused tail then adds the computed shared output instead of its shared units)
       const bool with_sdn = fuse_dn && sh8;
-      rc = launch_route_gate_up(a, n, logits, ld, wts->router_bias, c.n_experts, c.top_k, c.scoring,
-                                c.n_group, c.topk_group, c.norm_topk, c.routed_scale, has_sg, idx,
-                                wv, sg, tile_map, tiles_small, sorted, inv, stream,
-                                with_sdn ? &sdn : nullptr);
-      if (rc == 1)
-        rc = launch_route_gate_up(a, n, logits, ld, wts->router_bias, c.n_experts, c.top_k,
-                                  c.scoring, c.n_group, c.topk_group, c.norm_topk, c.routed_scale,
-                                  has_sg, idx, wv, sg, tile_map, tiles_small, sorted, inv, stream);
+      int r = launch_route_gate_up(a, n, logits, ld, wts->router_bias, c.n_experts, c.top_k, c.scoring,
+                                   c.n_group, c.topk_group, c.norm_topk, c.routed_scale, has_sg, idx,
+                                   wv, sg, tile_map, tiles_small, sorted, inv, stream,
+                                   with_sdn ? &sdn : nullptr);
+      if (r == 1)
+        r = launch_route_gate_up(a, n, logits, ld, wts->router_bias, c.n_experts, c.top_k,
+                                 c.scoring, c.n_group, c.topk_group, c.norm_topk, c.routed_scale,
+                                 has_sg, idx, wv, sg, tile_map, tiles_small, sorted, inv, stream);
       else
-        sdn_in_gate_up = with_sdn && rc == 0;
-    } else if (fuse_dn && sh8 && !hybrid && gfmt == FMT_INT4 && !tail) {
+        sdn_in_gate_up = with_sdn && r == 0;
+      return r;
+    }
+    if (fuse_dn && sh8 && !hybrid && gfmt == FMT_INT4 && !tail) {
       a.tile_map = reinterpret_cast<const int4*>(tile_map);
-      rc = launch_gate_up_shared_down(a, tiles_small, shared_down_args(), stream);
-      if (rc == 1) rc = routed(a, gfmt, EPI_SWIGLU, x16, x_sinv);
-      else sdn_in_gate_up = (rc == 0);
-    } else {
-      rc = routed(a, gfmt, EPI_SWIGLU, x16, x_sinv);
+      const int r = launch_gate_up_shared_down(a, tiles_small, shared_down_args(), stream);
+      if (r != 1) {
+        sdn_in_gate_up = (r == 0);
+        return r;
+      }
     }
-    if (rc) return rc;
-    if (hybrid && aux) {   // h complete (cold rows from the auxiliary stream) before its fp16 copy
-      rc = link(aux->cold, aux->s, stream, "cold gate_up");
-      if (rc) return rc;
-    }
-  }
-  // 6-7. slot-major decode with a shared expert and one int4 down stack: routed down, shared
-  // down and combine in one launch per 16 output features (the down output stays on chip)
-  if (slot_major && fuse_dn && !mixed && dfmt == FMT_INT4 &&
-      down_combine_fits(n, c.top_k, c.hidden, c.inter, c.shared_inter)) {
-    if (sdn_in_gate_up)
-      return launch_down_combine(h, idx, wv, has_sg ? sg : nullptr, n, c.top_k, c.hidden, c.inter,
-                                 wts->dn_codes, wts->dn_sb, nullptr, 0, nullptr, nullptr, sfmt,
-                                 resid, y, stream, sh_out);
-    return launch_down_combine(h, idx, wv, has_sg ? sg : nullptr, n, c.top_k, c.hidden, c.inter,
-                               wts->dn_codes, wts->dn_sb, sh_h, c.shared_inter, sh_dn_w,
-                               sh8 ? wts->sh_dn_sb : nullptr, sfmt, resid, y, stream);
-  }
+    return routed(a, gfmt, EPI_SWIGLU, x16, x_sinv, cls);
+  };
   // 6. routed down -> d (sorted order)
-  {
+  auto down = [&](ExpertClass cls) -> int {
     QmmArgs a{};
     a.act = h; a.act_rows = mc; a.slot_div = 1; a.n_slots = mc;
     a.offsets = offsets; a.tile_off = tile_off; a.n_experts = c.n_experts;
     a.K = c.inter; a.n_rows = c.hidden; a.codes = wts->dn_codes; a.sb = wts->dn_sb;
     a.row_exp = fp16_large_fmt(dfmt) ? wts->dn_rexp : nullptr;
     a.out = d; a.ld_out = c.hidden;
-    if (f16_h) {
-      rc = launch_act_to_f16(h, mc, c.inter, h16, h_sinv, stream);
-      if (rc) return rc;
+    if (cls == kHotExperts && f16_h) {
+      const int r = launch_act_to_f16(h, mc, c.inter, h16, h_sinv, hstream,
+                                      reinterpret_cast<const int4*>(tile_map_big), hot_bound);
+      if (r) return r;
     }
-    if (hybrid && aux) {   // the cold down reads bf16 h, complete since the cold gate_up join
-      rc = link(aux->hready, stream, aux->s, "h to auxiliary stream");
-      if (rc) return rc;
+    if (!mixed) return routed(a, dfmt, EPI_BF16, h16, h_sinv, cls);
+    for (int i = 0; i < mixed->n_stacks; ++i) {
+      const qmoe_stack_t& st = mixed->stacks[i];
+      if (st.proj != QMOE_PROJ_DOWN) continue;
+      a.codes = st.codes; a.sb = st.sb; a.expert_map = st.expert_slot; a.row_exp = st.row_exp;
+      const int r = routed(a, kernel_fmt(st.format), EPI_BF16, h16, h_sinv, cls);
+      if (r) return r;
     }
-    if (mixed) {
-      for (int i = 0; i < mixed->n_stacks; ++i) {
-        const qmoe_stack_t& st = mixed->stacks[i];
-        if (st.proj != QMOE_PROJ_DOWN) continue;
-        a.codes = st.codes; a.sb = st.sb; a.expert_map = st.expert_slot; a.row_exp = st.row_exp;
-        rc = routed(a, kernel_fmt(st.format), EPI_BF16, h16, h_sinv);
-        if (rc) return rc;
-      }
-    } else {
-      rc = routed(a, dfmt, EPI_BF16, h16, h_sinv);
-      if (rc) return rc;
+    return 0;
+  };
+  if (hybrid) {
+    // two chains, no event between them; enqueued in turn so that neither stream waits for the host
+    if (f16_acts && aux && hstream == stream) {   // the fp16 copy of x, made on the auxiliary stream at the fork
+      const hipError_t err = hipStreamWaitEvent(stream, aux->xready, 0);
+      if (err != hipSuccess) return fail(std::string("forward: x16 wait: ") + hipGetErrorString(err));
     }
+    rc = gate_up(kColdExperts);
+    if (!rc) rc = gate_up(kHotExperts);
+    if (!rc) rc = down(kColdExperts);
+    if (!rc) rc = down(kHotExperts);
+    if (rc) return rc;
+  } else {
+    rc = gate_up(kAllExperts);
+    if (rc) return rc;
+    // 6-7. slot-major decode with a shared expert and one int4 down stack: routed down, shared
+    // down and combine in one launch per 16 output features (the down output stays on chip)
+    if (slot_major && fuse_dn && !mixed && dfmt == FMT_INT4 &&
+        down_combine_fits(n, c.top_k, c.hidden, c.inter, c.shared_inter)) {
+      if (sdn_in_gate_up)
+        return launch_down_combine(h, idx, wv, has_sg ? sg : nullptr, n, c.top_k, c.hidden, c.inter,
+                                   wts->dn_codes, wts->dn_sb, nullptr, 0, nullptr, nullptr, sfmt,
+                                   resid, y, stream, sh_out);
+      return launch_down_combine(h, idx, wv, has_sg ? sg : nullptr, n, c.top_k, c.hidden, c.inter,
+                                 wts->dn_codes, wts->dn_sb, sh_h, c.shared_inter, sh_dn_w,
+                                 sh8 ? wts->sh_dn_sb : nullptr, sfmt, resid, y, stream);
+    }
+    rc = down(kAllExperts);
+    if (rc) return rc;
   }
   if (shared_down_late) {
     rc = shared_down();

@@ -1126,52 +1126,75 @@ __global__ void __launch_bounds__(kWdThreads, 1) qmm_wide_int3_kernel(QmmArgs a)
 }
 
 // ---------------------------------------------------------------- fp16 activation copy
-// One wavefront per row, the row held in registers (RPL 16-byte pieces per lane): absmax by a
+// One wavefront per RW rows, held in registers (RPL 16-byte pieces per lane and row): absmax by a
 // wavefront reduction, then act16 = fp16(act * 2^(14 - e)) with 2^(e-1) <= absmax < 2^e, so every
 // value sits below 2^14 and all bf16 values within 2^28 of the row maximum convert exactly.
 // row_sinv = 2^(e - 14) undoes it on the product (a power of two: exact). The maximum is exact in
 // any order, so the result does not depend on the launch shape.
-template <int RPL>
+// With tiles, launch row i is row i % 128 of m-tile i / 128 (-1: past its end). Four rows per
+// wavefront there: most tiles are partly filled, and a wavefront for every row of every tile costs
+// more than the rows (c2 2000 tokens: 86 thousand wavefronts for 19 thousand rows).
+__device__ __forceinline__ int64_t act16_row(int64_t i, int64_t rows, const int4* tiles) {
+  if (!tiles) return i < rows ? i : -1;
+  const int4 t = tiles[i / kLargeMTile];
+  const int r = static_cast<int>(i % kLargeMTile);
+  return (t.x >= 0 && r < t.z) ? t.y + r : -1;
+}
+template <int RPL, int RW>
 __global__ void __launch_bounds__(256) act_to_f16_kernel(const uint16_t* __restrict__ act, int K,
                                                          int64_t rows,
                                                          uint16_t* __restrict__ act16,
-                                                         float* __restrict__ row_sinv) {
+                                                         float* __restrict__ row_sinv,
+                                                         const int4* __restrict__ tiles) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;   // whole wavefront
-  const u32x4* src = reinterpret_cast<const u32x4*>(act + row * K);
+  // (a wavefront's rows lie in one tile: RW divides kLargeMTile)
+  const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * RW;
+  const int64_t row0 = act16_row(i0, rows, tiles);
+  if (row0 < 0) return;   // whole wavefront
   const int n8 = K / 8;
-  u32x4 v[RPL];
-  float m = 0.f;
+  u32x4 v[RW][RPL];
+  bool on[RW];
 #pragma unroll
-  for (int i = 0; i < RPL; ++i) {
-    const int c = lane + 64 * i;
-    v[i] = (c < n8) ? src[c] : u32x4{0u, 0u, 0u, 0u};
+  for (int w = 0; w < RW; ++w) {
+    on[w] = (w == 0) || act16_row(i0 + w, rows, tiles) >= 0;
+    const u32x4* src = reinterpret_cast<const u32x4*>(act + (row0 + (on[w] ? w : 0)) * K);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      m = fmaxf(m, fabsf(bf16lo_to_f32(v[i][j])));
-      m = fmaxf(m, fabsf(bf16hi_to_f32(v[i][j])));
+    for (int i = 0; i < RPL; ++i) {
+      const int c = lane + 64 * i;
+      v[w][i] = (c < n8) ? src[c] : u32x4{0u, 0u, 0u, 0u};
     }
   }
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  int ex = 0;
-  if (m > 0.f && m <= 3.4e38f) frexpf(m, &ex);   // m = f * 2^ex, f in [0.5, 1)
-  const int sh = (m > 0.f && m <= 3.4e38f) ? 14 - ex : 0;
-  if (lane == 0) row_sinv[row] = ldexpf(1.0f, -sh);
-  u32x4* dst = reinterpret_cast<u32x4*>(act16 + row * K);
+  for (int w = 0; w < RW; ++w) {
+    if (!on[w]) break;
+    float m = 0.f;
 #pragma unroll
-  for (int i = 0; i < RPL; ++i) {
-    const int c = lane + 64 * i;
-    if (c < n8) {
-      u32x4 o;
+    for (int i = 0; i < RPL; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f16x2_t h = {static_cast<_Float16>(ldexpf(bf16lo_to_f32(v[i][j]), sh)),
-                           static_cast<_Float16>(ldexpf(bf16hi_to_f32(v[i][j]), sh))};
-        o[j] = __builtin_bit_cast(uint32_t, h);
+        m = fmaxf(m, fabsf(bf16lo_to_f32(v[w][i][j])));
+        m = fmaxf(m, fabsf(bf16hi_to_f32(v[w][i][j])));
       }
-      dst[c] = o;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    int ex = 0;
+    if (m > 0.f && m <= 3.4e38f) frexpf(m, &ex);   // m = f * 2^ex, f in [0.5, 1)
+    const int sh = (m > 0.f && m <= 3.4e38f) ? 14 - ex : 0;
+    if (lane == 0) row_sinv[row0 + w] = ldexpf(1.0f, -sh);
+    u32x4* dst = reinterpret_cast<u32x4*>(act16 + (row0 + w) * K);
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+      const int c = lane + 64 * i;
+      if (c < n8) {
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f16x2_t h = {static_cast<_Float16>(ldexpf(bf16lo_to_f32(v[w][i][j]), sh)),
+                             static_cast<_Float16>(ldexpf(bf16hi_to_f32(v[w][i][j]), sh))};
+          o[j] = __builtin_bit_cast(uint32_t, h);
+        }
+        dst[c] = o;
+      }
     }
   }
 }
@@ -1179,9 +1202,11 @@ __global__ void __launch_bounds__(256) act_to_f16_kernel(const uint16_t* __restr
 // Rows longer than 8192: one workgroup per row, the row read twice (absmax, then convert).
 __global__ void __launch_bounds__(256) act_to_f16_wide_kernel(const uint16_t* __restrict__ act, int K,
                                                          uint16_t* __restrict__ act16,
-                                                         float* __restrict__ row_sinv) {
+                                                         float* __restrict__ row_sinv, int64_t rows,
+                                                         const int4* __restrict__ tiles) {
   __shared__ float red[4];
-  const int64_t row = blockIdx.x;
+  const int64_t row = act16_row(blockIdx.x, rows, tiles);
+  if (row < 0) return;   // whole workgroup
   const u32x4* src = reinterpret_cast<const u32x4*>(act + row * K);
   const int n8 = K / 8;
   float m = 0.f;
@@ -1217,23 +1242,27 @@ __global__ void __launch_bounds__(256) act_to_f16_wide_kernel(const uint16_t* __
 }
 
 int launch_act_to_f16(const uint16_t* act, int64_t rows, int K, uint16_t* act16, float* row_sinv,
-                      hipStream_t stream) {
+                      hipStream_t stream, const int4* tiles, int64_t n_tiles) {
+  if (tiles) rows = n_tiles * kLargeMTile;   // launch rows: every row of every tile
   if (rows <= 0) return 0;
   if (K % 8) return fail("act_to_f16: K % 8 == 0 required");
   if (K > 8 * 64 * 16) {
     if (rows > 0x7fffffff) return fail("act_to_f16: too many rows");
-    act_to_f16_wide_kernel<<<static_cast<unsigned>(rows), 256, 0, stream>>>(act, K, act16, row_sinv);
+    act_to_f16_wide_kernel<<<static_cast<unsigned>(rows), 256, 0, stream>>>(act, K, act16, row_sinv, rows, tiles);
     return check_launch("act_to_f16");
   }
   if (rows > (int64_t(1) << 32)) return fail("act_to_f16: too many rows");
-  const unsigned grid = static_cast<unsigned>((rows + 3) / 4);
   const int rpl = (K / 8 + 63) / 64;   // 16-byte pieces per lane
-#define QMOE_A16(R) act_to_f16_kernel<R><<<grid, 256, 0, stream>>>(act, K, rows, act16, row_sinv)
-  if (rpl <= 2) QMOE_A16(2);
-  else if (rpl <= 4) QMOE_A16(4);
-  else if (rpl <= 8) QMOE_A16(8);
-  else if (rpl <= 14) QMOE_A16(14);
-  else QMOE_A16(16);
+#define QMOE_A16(R, RW)                                                                              \
+  act_to_f16_kernel<R, RW><<<static_cast<unsigned>((rows + 4 * RW - 1) / (4 * RW)), 256, 0, stream>>>( \
+      act, K, rows, act16, row_sinv, tiles)
+  if (tiles && rpl <= 2) QMOE_A16(2, 4);
+  else if (tiles && rpl <= 4) QMOE_A16(4, 4);
+  else if (rpl <= 2) QMOE_A16(2, 1);
+  else if (rpl <= 4) QMOE_A16(4, 1);
+  else if (rpl <= 8) QMOE_A16(8, 1);
+  else if (rpl <= 14) QMOE_A16(14, 1);
+  else QMOE_A16(16, 1);
 #undef QMOE_A16
   return check_launch("act_to_f16");
 }
@@ -1657,6 +1686,7 @@ int launch_qmm(const QmmArgs& a, int fmt, int epi, int regime, int64_t mtile_bou
                hipStream_t stream) {
   if (a.K <= 0 || a.n_rows <= 0) return fail("qmm: empty problem");
   if (mtile_bound <= 0) return 0;
+  if (regime == kRegimeDense) return launch_dense(a, fmt, epi, stream);
   if (mtile_bound > 65535) return fail("qmm: too many m-tiles for one launch");
   if (a.expert_map && !fmt_quant(fmt))
     return fail("qmm: an expert map needs int3/int4/int6 weights");

@@ -308,8 +308,12 @@ __device__ __forceinline__ u32x4 dense_bf16(const DenseFrag<FMT>& f) {
 }
 enum { EPI_SWIGLU = 0, EPI_BF16 = 1, EPI_F32 = 2 };
 
+// regime: QMOE_REGIME_SMALL, QMOE_REGIME_LARGE, or kRegimeDense (dense products of batches above
+// the decode sizes, qmm_dense_kernel; mtile_bound unused).
+constexpr int kRegimeDense = 3;
 int launch_qmm(const QmmArgs& a, int fmt, int epi, int regime, int64_t mtile_bound,
                hipStream_t stream);
+int launch_dense(const QmmArgs& a, int fmt, int epi, hipStream_t stream);   // (dense.hip)
 // Chunk count of the small-regime bf16 products over K: ~8 32-deep steps per chunk, one
 // wavefront per chunk, chunk sums added in chunk order.
 inline int bf16_chunks(int K) {
@@ -338,9 +342,10 @@ int launch_combine_shared(const uint16_t* d, const int32_t* inv, const float* w,
 int launch_expand_int8(const uint32_t* codes, const uint16_t* sb, int64_t rows, int K,
                        uint16_t* out, hipStream_t stream);
 // act [rows][K] bf16 -> act16 fp16 with a per-row power-of-two scale (exact for bf16 values
-// within 2^28 of the row's largest magnitude); row_sinv[r] = the inverse scale.
+// within 2^28 of the row's largest magnitude); row_sinv[r] = the inverse scale. With tiles (n_tiles
+// m-tile descriptors of at most kLargeMTile rows), only the rows of those tiles.
 int launch_act_to_f16(const uint16_t* act, int64_t rows, int K, uint16_t* act16, float* row_sinv,
-                      hipStream_t stream);
+                      hipStream_t stream, const int4* tiles = nullptr, int64_t n_tiles = 0);
 inline size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 inline size_t act16_ws_bytes(int64_t rows, int K) {
   return align256(static_cast<size_t>(rows) * K * 2) + align256(static_cast<size_t>(rows) * 4);
@@ -364,10 +369,11 @@ int launch_awq_prescale_split(const uint16_t* x, const int32_t* sorted, const in
                               int split_rows, uint16_t* xgu, uint16_t* x16, float* x_sinv,
                               hipStream_t stream);
 // h[m] = bf16(glu(g, u) / s_dn[e]) over gu [mc][2I] (gate | up, bf16) with s_dn bf16 [E][I];
-// s_dn NULL: h[m] = bf16(glu(g, u)) (offsets unused).
+// s_dn NULL: h[m] = bf16(glu(g, u)). cls: the rows of all experts, or only of those with at most
+// (cold) or more than (hot) split_rows rows.
 int launch_awq_glu(const uint16_t* gu, const int32_t* offsets, int E, int64_t mc, int I,
                    const uint16_t* s_dn, int act, float alpha, float limit, uint16_t* h,
-                   hipStream_t stream);
+                   hipStream_t stream, int cls, int split_rows);
 // For H % 32 == 0 the sum of squares follows the canonical order that the fused-norm pair launch
 // also follows: H cut into bf16_chunks(H) chunks of 32-wide steps; within a chunk, lane group g
 // (0..3) sums the elements 32 s + 8 g + j (steps s in order, j = 0..7 in order) with fmaf from
@@ -413,7 +419,16 @@ constexpr int kSyncStride = 64;
 constexpr int kSmallMTile = 16;
 constexpr int kLargeMTile = 128;
 // Large-M (prefill) regime: experts routed more rows than this use 128-row tiles on the large
-// kernel, the others 16-row tiles on the small kernel.
-constexpr int kHybridSplitRows = 16;
+// kernel, the others 16-row tiles on the small kernel. Experts of 17 to 32 rows are cheaper as two
+// 16-row tiles (the second one's weights come from L2) while there are few of them, up to about 14
+// rows per expert on average: the large kernel's chain of a few latency-bound workgroups then
+// outlasts the cold experts' (c1 391 tokens 207 us per layer against 220, c2 600 skewed 699 / 724);
+// from 18 rows on they are most of the experts and the large kernel streams them once (c2 1000
+// tokens 982 / 1331).
+inline bool few_hot(int64_t mc, int64_t n_experts) { return mc <= 14 * n_experts; }
+inline int hybrid_split_rows(int64_t mc, int64_t n_experts) { return few_hot(mc, n_experts) ? 32 : 16; }
+// Which experts a launch of the routed products covers: all (one regime), or the hybrid regime's
+// cold or hot ones.
+enum ExpertClass { kAllExperts = 0, kColdExperts = 1, kHotExperts = 2 };
 
 }  // namespace qmoe

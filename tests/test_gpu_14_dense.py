@@ -1,0 +1,68 @@
+"""GPU tier: the dense products of batches above the decode sizes (dense.hip `qmm_dense_kernel`: router
+logits and the shared expert over 64-token x 64-row tiles) and the two-chain hybrid regime around
+them, against the oracle.
+
+The shapes sit where the kernel's tiling can go wrong: hidden and shared sizes for each number of
+wavefronts that cut K (1, 2, 4 and 8, with stages that do not divide evenly), weight-row blocks that
+do not fill a workgroup, router rows past the experts, the last token block with 1, 63 and 64 rows,
+more tokens than weight rows (the other tile order), and hidden sizes off the large kernel's 256
+(no hybrid regime). Shared weights are scaled up so that they carry most of the output. Bars: the
+BASELINE gates (tests/_util.assert_close).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import moe as om
+from quanta_amd import synth
+from quanta_amd.moe import qwen35_moe
+from quanta_amd.quant import quantize_affine
+from tests._util import assert_close, f64, oracle_params_from_torch
+
+pytestmark = pytest.mark.gpu
+
+SHARED = ("shared_gate_proj", "shared_up_proj", "shared_down_proj")
+
+
+@pytest.mark.parametrize("bits", [8, 16])
+@pytest.mark.parametrize("N,H,Is,E", [(257, 256, 128, 8), (319, 384, 640, 16), (320, 512, 1152, 40),
+                                      (450, 1024, 256, 64), (321, 2176, 512, 96), (700, 256, 384, 255)])
+def test_dense_products_vs_oracle(gpu, N, H, Is, E, bits):
+    s = synth.scaled_spec("c1", hidden_size=H, num_experts=E, num_experts_per_tok=2,
+                          moe_intermediate_size=128, shared_expert_intermediate_size=Is)
+    p = synth.make_layer(s, device=gpu, seed=N)
+    for key in SHARED:
+        w = (p[key].float() * 8.0).to(torch.bfloat16)
+        if bits == 8:
+            pk, sc, bi = quantize_affine(w, 8, group_size=64)
+            w = {"packed": pk, "scale": sc, "bias": bi, "group_size": 64, "bits": 8}
+        p[key] = w
+    x = synth.make_inputs(s, N, device=gpu, seed=3 + N)
+    y = qwen35_moe(x[None], p, s.cfg)[0]
+    _, it = om.moe_forward(f64(x), oracle_params_from_torch(p), k=2, inter=128)
+    assert_close(f64(y), it["y_exact"], f"dense N={N} H={H} Is={Is} E={E} int{bits}")
+
+
+@pytest.mark.parametrize("E,N", [(64, 300), (32, 400), (8, 300)])
+def test_two_chains_repeat_bit_for_bit(gpu, E, N):
+    """The hot and cold experts' chains run on two streams over disjoint rows: repeated calls on
+    one workspace, on two streams, give the same bits (mean rows per expert 9, 25 and 75: the cold
+    chain, then the hot one on the caller's stream)."""
+    s = synth.scaled_spec("c1", hidden_size=512, num_experts=E, num_experts_per_tok=2,
+                          moe_intermediate_size=256, shared_expert_intermediate_size=256)
+    p = synth.make_layer(s, device=gpu, seed=E)
+    x = synth.make_inputs(s, N, device=gpu, seed=N)[None]
+    want = qwen35_moe(x, p, s.cfg)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for i in range(6):
+        if i % 2:
+            with torch.cuda.stream(side):
+                y = qwen35_moe(x, p, s.cfg)
+            side.synchronize()
+        else:
+            y = qwen35_moe(x, p, s.cfg)
+            torch.cuda.synchronize()
+        assert torch.equal(y, want), i
