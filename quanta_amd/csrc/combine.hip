@@ -442,9 +442,9 @@ static WsLayout ws_layout(const qmoe_config_t& c, int64_t N) {
   // (the shared expert's SwiGLU output, or with the decode dataflow launch its [gate | up] rows)
   L.sh_h = take(static_cast<size_t>(N) * (c.shared_inter > 0 ? 2 * c.shared_inter : 0) * 2);
   L.sh_out = take(static_cast<size_t>(N) * (c.shared_inter > 0 ? c.hidden : 0) * 2);
-  // int8 shared expert above the decode sizes: its weights expanded to tiled bf16 for the
-  // large-M kernel (gate|up [2 Is, H] then down [H, Is])
-  L.sh_w16 = take((expand_gu(c, N) || expand_dn(c, N)) ? static_cast<size_t>(3) * c.shared_inter * c.hidden * 2 : 0);
+  // int8 shared expert above the decode sizes: room for its weights expanded to tiled bf16 for the
+  // large-M kernel (gate|up [2 Is, H] then down [H, Is]; expand_gu, expand_dn)
+  L.sh_w16 = take(shared_int8(c) && large_ok(c, N) ? static_cast<size_t>(3) * c.shared_inter * c.hidden * 2 : 0);
   // fp16 per-row-scaled activation copies for the large-M int4 regime (AWQ: of the gate's and
   // the up projection's prescaled rows, [2][mc])
   const int64_t x16_rows = c.awq ? 2 * mc : N;
