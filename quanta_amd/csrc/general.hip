@@ -11,10 +11,11 @@
 //            shared weights' dtype                                     (:145-151)
 //   y = cast_x(routed + shared)                                        (:201-202)
 // as the reference's own float32 parity gates run it (parity/qwen35_forward_test.py:213-271:
-// hidden 32, group size 32, float32 throughout). Every matrix-vector product is one wavefront per
-// output (lanes stride K, a fixed-order wavefront sum, fp32 accumulation); the affine weight
-// s*q + b is evaluated in fp32 per element from the LSB-first packed code stream. These shapes are
-// small (the parity configs); the fast path serves the bf16 g64 production formats.
+// hidden 32, group size 32, float32 throughout). Four launches (six with a shared expert): router, top-k,
+// gate_up with its gated activation, down with the combine; one wavefront per output (fixed-order
+// wavefront sums, fp32 accumulation), the affine weight s*q + b evaluated in fp32 per element from
+// the LSB-first packed code stream. These shapes are small (the parity configs); the fast path
+// serves the bf16 g64 production formats.
 #include <math.h>
 
 #include "qmoe_internal.h"
@@ -35,98 +36,259 @@ __device__ __forceinline__ void gen_st(void* p, int64_t i, float v, int dt) {
   else static_cast<uint16_t*>(p)[i] = f32_to_bf16(v);
 }
 
-// out[r][col0 + o] = sum_k a(r, k) * W_e(r)[o][k]: a = the activation row r / row_div, rounded to
-// act_round when that differs from its dtype (the reference's cast to the weights' dtype); W a
-// dense [E][n_out][K] stack or affine codes (bits, group gs, scale/bias [E][n_out][K/gs]).
+// Weights of the products: a dense [rows][K] stack (BITS 0; `dense_dt`) or affine codes with a scale
+// and a bias per group of 2^gshift along K.
+struct GenW {
+  const uint32_t* packed;
+  const void* scale;
+  const void* bias;
+  const void* dense;
+  int sb_dt, dense_dt, gshift, K;
+};
+
+// Every product is one wavefront per output (or per few outputs over the same activations): lane l
+// takes the 8-element pieces l, l + 64, ... of K, so that a row of 512 is one round of loads. At
+// these sizes the launch is a chain of dependent loads; element-strided lanes took eight rounds.
+// Elements 8c .. 8c + 7 of activation row `base` (element offset), rounded to act_round when that
+// differs from their dtype (the reference's cast to the weights' dtype); 0 past K.
+template <bool VEC>
+__device__ __forceinline__ void gen_x8(const void* act, int64_t base, int c, int K, int dt, int round,
+                                       float (&x)[8]) {
+  if (VEC) {   // (rows 16-byte aligned, K % 8 == 0)
+    if (dt == QMOE_DT_F32) {
+      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(static_cast<const float*>(act) + base + 8 * c);
+      const f32x4_t lo = p[0], hi = p[1];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[j] = lo[j];
+        x[4 + j] = hi[j];
+      }
+    } else {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(act) + base + 8 * c);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[2 * j] = bf16lo_to_f32(v[j]);
+        x[2 * j + 1] = bf16hi_to_f32(v[j]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = (8 * c + j < K) ? gen_ld(act, base + 8 * c + j, dt) : 0.f;
+  }
+  if (round != dt) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = gen_round(x[j], round);
+  }
+}
+
+// acc + x . W[row][8c .. 8c + 7], the affine weight fma(s, q, b) formed in fp32 per element. Eight
+// codes of any width start on a byte and span at most two words.
+template <int BITS, bool VEC>
+__device__ __forceinline__ float gen_dot8(const GenW& w, int64_t row, int c, const float (&x)[8], float acc) {
+  if constexpr (BITS > 0) {
+    const uint32_t* p = w.packed + row * (static_cast<int64_t>(w.K) * BITS / 32);
+    const int bit = 8 * BITS * c, sh = bit & 31;
+    uint64_t v = p[bit >> 5];
+    if (sh + 8 * BITS > 32) v |= static_cast<uint64_t>(p[(bit >> 5) + 1]) << 32;
+    v >>= sh;
+    const int64_t g = row * (w.K >> w.gshift) + ((8 * c) >> w.gshift);
+    const float s = gen_ld(w.scale, g, w.sb_dt), b = gen_ld(w.bias, g, w.sb_dt);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t q = static_cast<uint32_t>(v >> (j * BITS)) & ((1u << BITS) - 1u);
+      acc = fmaf(x[j], fmaf(s, static_cast<float>(q), b), acc);
+    }
+  } else {
+    float y[8];
+    gen_x8<VEC>(w.dense, row * w.K, c, w.K, w.dense_dt, w.dense_dt, y);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc = fmaf(x[j], y[j], acc);
+  }
+  return acc;
+}
+
+template <int M>
+__device__ __forceinline__ void gen_wave_sum(float (&v)[M]) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < M; ++i) v[i] += __shfl_xor(v[i], off);
+}
+
+// out[r][col0 + o] = a(r) . W[o], a = the activation row r (the router's and the shared expert's
+// down products).
 struct GenMv {
   const void* act;
   int act_dt, act_round;     // QMOE_DT_*; act_round: the dtype the activation is cast to first
-  int64_t act_rows;
-  int K;
-  const int32_t* row_expert;  // [rows] expert of each output row (nullable: expert 0)
-  int row_div;
   int64_t rows;
   int n_out;
-  const uint32_t* packed;     // affine codes (nullable: dense)
-  const void* scale;
-  const void* bias;
-  int bits, gs, sb_dt;
-  const void* dense;
-  int dense_dt;
+  GenW w;
   void* out;
   int out_dt;
   int64_t ld_out;
   int col0;
 };
 
+template <bool VEC>
 __global__ void __launch_bounds__(256) gen_matvec_kernel(GenMv a) {
   const int lane = threadIdx.x & 63;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (gid >= a.rows * a.n_out) return;   // whole wavefronts exit together; no barriers below
   const int64_t r = gid / a.n_out;
   const int o = static_cast<int>(gid - r * a.n_out);
-  const int e = a.row_expert ? a.row_expert[r] : 0;
-  const int64_t ar = r / a.row_div;
-  float acc = 0.f;
-  if (ar < a.act_rows && e >= 0) {
-    const int64_t wrow = static_cast<int64_t>(e) * a.n_out + o;
-    const int64_t abase = ar * a.K;
-    const int64_t words = static_cast<int64_t>(a.K) * a.bits / 32;
-    const uint32_t mask = (1u << a.bits) - 1u;
-    for (int k = lane; k < a.K; k += 64) {
-      float xv = gen_ld(a.act, abase + k, a.act_dt);
-      if (a.act_round != a.act_dt) xv = gen_round(xv, a.act_round);
-      float wv;
-      if (a.packed) {
-        const int64_t bit = static_cast<int64_t>(k) * a.bits;
-        const uint32_t* p = a.packed + wrow * words + bit / 32;
-        const int sh = static_cast<int>(bit & 31);
-        uint32_t c = p[0] >> sh;
-        if (sh + a.bits > 32) c |= p[1] << (32 - sh);
-        const int64_t g = wrow * (a.K / a.gs) + k / a.gs;
-        wv = fmaf(gen_ld(a.scale, g, a.sb_dt), static_cast<float>(c & mask), gen_ld(a.bias, g, a.sb_dt));
-      } else {
-        wv = gen_ld(a.dense, wrow * a.K + k, a.dense_dt);
-      }
-      acc = fmaf(xv, wv, acc);
-    }
+  float acc[1] = {0.f};
+  for (int c = lane; 8 * c < a.w.K; c += 64) {
+    float x[8];
+    gen_x8<VEC>(a.act, r * a.w.K, c, a.w.K, a.act_dt, a.act_round, x);
+    acc[0] = gen_dot8<0, VEC>(a.w, o, c, x, acc[0]);
   }
+  gen_wave_sum(acc);
+  if (lane == 0) gen_st(a.out, r * a.ld_out + a.col0 + o, acc[0], a.out_dt);
+}
+
+// h[r][i] = glu(g, u) in dtype dt: g and u the products of activation row r / row_div with weight
+// rows e(r) n2 + i and that + up (or row i of w_up), each rounded to dt as the reference's
+// materialised gate_up is.
+struct GenGu {
+  const void* act;
+  int act_dt, act_round;
+  const int32_t* row_expert;  // [rows] expert of each output row (nullable: expert 0)
+  int row_div;
+  int64_t rows;
+  int n, n2, up;
+  GenW w, w_up;
+  void* h;
+  int dt, glu;
+  float alpha, limit;
+};
+
+template <int BITS, bool VEC>
+__global__ void __launch_bounds__(256) gen_gate_up_kernel(GenGu a) {
+  const int lane = threadIdx.x & 63;
+  const int64_t gid = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (gid >= a.rows * a.n) return;
+  const int64_t r = gid / a.n;
+  const int i = static_cast<int>(gid - r * a.n);
+  const int e = a.row_expert ? a.row_expert[r] : 0;   // (-1: no expert, zeros)
+  const int64_t row = static_cast<int64_t>(e) * a.n2 + i;
+  const int64_t base = r / a.row_div * a.w.K;
+  float v[2] = {0.f, 0.f};
+  for (int c = lane; e >= 0 && 8 * c < a.w.K; c += 64) {
+    float x[8];
+    gen_x8<VEC>(a.act, base, c, a.w.K, a.act_dt, a.act_round, x);
+    v[0] = gen_dot8<BITS, VEC>(a.w, row, c, x, v[0]);
+    v[1] = gen_dot8<BITS, VEC>(a.w_up, row + a.up, c, x, v[1]);
+  }
+  gen_wave_sum(v);
+  if (lane == 0)
+    gen_st(a.h, r * a.n + i, glu_f(gen_round(v[0], a.dt), gen_round(v[1], a.dt), a.glu, a.alpha, a.limit), a.dt);
+}
+
+// y[t][j] = cast_x(sum_s f32(d_s) * w[t][s] + f32(sh[t][j]) * sg[t]), d_s = h[t*k+s] . W_e[j] rounded
+// to dtype dt (the reference's materialised down output), slots in order.
+struct GenDn {
+  const void* h;
+  int dt;
+  const int32_t* idx;
+  const float* wt;
+  int64_t N;
+  int k, H;
+  GenW w;
+  const void* sh;
+  int sh_dt;
+  const float* sg;
+  void* y;
+  int y_dt;
+};
+
+template <int BITS, bool VEC>
+__global__ void __launch_bounds__(256) gen_down_combine_kernel(GenDn a) {
+  const int lane = threadIdx.x & 63;
+  const int64_t gid = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (gid >= a.N * a.H) return;
+  const int64_t t = gid / a.H;
+  const int j = static_cast<int>(gid - t * a.H);
+  float out = 0.f;
+  constexpr int SB = 4;   // slots whose loads and sums run together
+  for (int s0 = 0; s0 < a.k; s0 += SB) {
+    float v[SB];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-  if (lane == 0) gen_st(a.out, r * a.ld_out + a.col0 + o, acc, a.out_dt);
+    for (int i = 0; i < SB; ++i) {
+      v[i] = 0.f;
+      if (s0 + i < a.k) {
+        const int64_t m = t * a.k + s0 + i;
+        const int e = a.idx[m];
+        const int64_t row = static_cast<int64_t>(e) * a.H + j;
+        for (int c = lane; e >= 0 && 8 * c < a.w.K; c += 64) {
+          float x[8];
+          gen_x8<VEC>(a.h, m * a.w.K, c, a.w.K, a.dt, a.dt, x);
+          v[i] = gen_dot8<BITS, VEC>(a.w, row, c, x, v[i]);
+        }
+      }
+    }
+    gen_wave_sum(v);
+#pragma unroll
+    for (int i = 0; i < SB; ++i)
+      if (s0 + i < a.k) out += gen_round(v[i], a.dt) * a.wt[t * a.k + s0 + i];
+  }
+  if (lane == 0) {
+    if (a.sh) out += gen_ld(a.sh, gid, a.sh_dt) * (a.sg ? a.sg[t] : 1.0f);
+    gen_st(a.y, gid, out, a.y_dt);
+  }
+}
+
+// 16-byte loads of activation and dense weight rows need whole 8-element pieces and aligned bases;
+// anything else (the caller's tensors may start anywhere) loads element by element.
+static bool gen_vec(int K, const void* a, const void* b = nullptr, const void* c = nullptr) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c);
+  return K % 8 == 0 && bits % 16 == 0;
+}
+
+static int gen_grid(int64_t waves, unsigned* grid) {
+  if ((waves + 3) / 4 > 0x7fffffff) return fail("general: product too large");
+  *grid = static_cast<unsigned>((waves + 3) / 4);
+  return 0;
 }
 
 static int gen_matvec(const GenMv& a, hipStream_t stream) {
-  const int64_t waves = a.rows * a.n_out;
-  if (waves <= 0) return 0;
-  if ((waves + 3) / 4 > 0x7fffffff) return fail("general: product too large");
-  gen_matvec_kernel<<<dim3(static_cast<unsigned>((waves + 3) / 4)), 256, 0, stream>>>(a);
+  unsigned grid;
+  if (int rc = gen_grid(a.rows * a.n_out, &grid)) return rc;
+  if (!grid) return 0;
+  if (gen_vec(a.w.K, a.act, a.w.dense)) gen_matvec_kernel<true><<<grid, 256, 0, stream>>>(a);
+  else gen_matvec_kernel<false><<<grid, 256, 0, stream>>>(a);
   return check_launch("general matvec");
 }
 
-// h[r][i] = glu(gu[r][i], gu[r][n + i]) in dtype dt (fp32 math, one rounding)
-__global__ void __launch_bounds__(256) gen_glu_kernel(const void* gu, void* h, int64_t rows, int n,
-                                                      int dt, int act, float alpha, float limit) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= rows * n) return;
-  const int64_t r = i / n, c = i - r * n;
-  const float g = gen_ld(gu, r * 2 * n + c, dt), u = gen_ld(gu, r * 2 * n + n + c, dt);
-  gen_st(h, i, glu_f(g, u, act, alpha, limit), dt);
+// launch KERNEL<bits, vec> for a code width (0: dense)
+#define QMOE_GEN(KERNEL, bits, vec, grid, stream, a)                                                          \
+  do {                                                                                                        \
+    switch (bits) {                                                                                           \
+      case 0: if (vec) KERNEL<0, true><<<grid, 256, 0, stream>>>(a); else KERNEL<0, false><<<grid, 256, 0, stream>>>(a); break; \
+      case 2: if (vec) KERNEL<2, true><<<grid, 256, 0, stream>>>(a); else KERNEL<2, false><<<grid, 256, 0, stream>>>(a); break; \
+      case 3: if (vec) KERNEL<3, true><<<grid, 256, 0, stream>>>(a); else KERNEL<3, false><<<grid, 256, 0, stream>>>(a); break; \
+      case 4: if (vec) KERNEL<4, true><<<grid, 256, 0, stream>>>(a); else KERNEL<4, false><<<grid, 256, 0, stream>>>(a); break; \
+      case 5: if (vec) KERNEL<5, true><<<grid, 256, 0, stream>>>(a); else KERNEL<5, false><<<grid, 256, 0, stream>>>(a); break; \
+      case 6: if (vec) KERNEL<6, true><<<grid, 256, 0, stream>>>(a); else KERNEL<6, false><<<grid, 256, 0, stream>>>(a); break; \
+      case 8: if (vec) KERNEL<8, true><<<grid, 256, 0, stream>>>(a); else KERNEL<8, false><<<grid, 256, 0, stream>>>(a); break; \
+      default: return fail("general: bits must be 2, 3, 4, 5, 6 or 8");                                       \
+    }                                                                                                         \
+  } while (0)
+
+static int gen_gate_up(const GenGu& a, int bits, hipStream_t stream) {
+  unsigned grid;
+  if (int rc = gen_grid(a.rows * a.n, &grid)) return rc;
+  if (!grid) return 0;
+  const bool vec = gen_vec(a.w.K, a.act, bits ? nullptr : a.w.dense, bits ? nullptr : a.w_up.dense);
+  QMOE_GEN(gen_gate_up_kernel, bits, vec, grid, stream, a);
+  return check_launch("general gate_up");
 }
 
-// y[t][j] = cast_x(sum_s f32(d[t*k+s][j]) * w[t][s] + f32(sh[t][j]) * sg[t])
-__global__ void __launch_bounds__(256) gen_combine_kernel(const void* d, int d_dt, const float* w,
-                                                          int N, int k, int H, const void* sh,
-                                                          int sh_dt, const float* sg, void* y,
-                                                          int y_dt) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= static_cast<int64_t>(N) * H) return;
-  const int64_t t = i / H, j = i - t * H;
-  float acc = 0.f;
-  for (int s = 0; s < k; ++s)
-    acc += gen_ld(d, (t * k + s) * H + j, d_dt) * w[t * k + s];
-  if (sh) acc += gen_ld(sh, t * H + j, sh_dt) * (sg ? sg[t] : 1.0f);
-  gen_st(y, i, acc, y_dt);
+static int gen_down_combine(const GenDn& a, int bits, hipStream_t stream) {
+  unsigned grid;
+  if (int rc = gen_grid(a.N * a.H, &grid)) return rc;
+  const bool vec = gen_vec(a.w.K, a.h, bits ? nullptr : a.w.dense);
+  QMOE_GEN(gen_down_combine_kernel, bits, vec, grid, stream, a);
+  return check_launch("general down + combine");
 }
 
 // The run-every-expert form (the reference's sparse=False oracle, moe.py:127-142): every token
@@ -148,7 +310,7 @@ __global__ void __launch_bounds__(256) gen_scatter_kernel(const int32_t* idx, co
 }
 
 struct GenLayout {
-  size_t logits, idx, w, sg, idx_all, w_all, gu, h, d, sgu, sh, so, total;
+  size_t logits, idx, w, sg, idx_all, w_all, h, sh, so, total;
 };
 static int dt_bytes(int dt) { return dt == QMOE_DT_F32 ? 4 : 2; }
 // The routed experts' compute dtype: a dense stack's own dtype (x is cast to it, moe.py:77); for
@@ -175,10 +337,7 @@ static GenLayout gen_layout(const qmoe_general_config_t& c, int64_t N) {
   L.sg = take(static_cast<size_t>(N) * 4);
   L.idx_all = take(c.dense_all ? static_cast<size_t>(mc) * 4 : 0);
   L.w_all = take(c.dense_all ? static_cast<size_t>(mc) * 4 : 0);
-  L.gu = take(static_cast<size_t>(mc) * 2 * c.inter * te);
   L.h = take(static_cast<size_t>(mc) * c.inter * te);
-  L.d = take(static_cast<size_t>(mc) * c.hidden * te);
-  L.sgu = take(static_cast<size_t>(N) * 2 * c.shared_inter * ts);
   L.sh = take(static_cast<size_t>(N) * c.shared_inter * ts);
   L.so = take(static_cast<size_t>(N) * c.hidden * ts);
   L.total = o;
@@ -256,14 +415,19 @@ extern "C" int qmoe_forward_general(const qmoe_general_config_t* cfg, const qmoe
   const int ld = E + 1;
 
   // router logits in f32 (column E: the shared expert's gate logit)
+  auto dense_w = [](const void* p, int dt, int K) {
+    GenW w{};
+    w.dense = p; w.dense_dt = dt; w.K = K;
+    return w;
+  };
   GenMv r{};
-  r.act = x; r.act_dt = c.x_dtype; r.act_round = c.x_dtype; r.act_rows = N; r.K = H;
-  r.row_div = 1; r.rows = N; r.n_out = E; r.dense = wts->gate; r.dense_dt = c.gate_dtype;
+  r.act = x; r.act_dt = c.x_dtype; r.act_round = c.x_dtype;
+  r.rows = N; r.n_out = E; r.w = dense_w(wts->gate, c.gate_dtype, H);
   r.out = logits; r.out_dt = QMOE_DT_F32; r.ld_out = ld;
   if ((rc = gen_matvec(r, st))) return rc;
   if (has_sg) {
     GenMv g = r;
-    g.n_out = 1; g.dense = wts->sh_expert_gate; g.dense_dt = c.shared_gate_dtype; g.col0 = E;
+    g.n_out = 1; g.w = dense_w(wts->sh_expert_gate, c.shared_gate_dtype, H); g.col0 = E;
     if ((rc = gen_matvec(g, st))) return rc;
   }
   rc = launch_topk(logits, ld, wts->router_bias, n, E, c.top_k, c.scoring, c.n_group, c.topk_group,
@@ -284,60 +448,46 @@ extern "C" int qmoe_forward_general(const qmoe_general_config_t* cfg, const qmoe
     ridx = ia;
     rw = wa;
   }
-  void* gu = base + L.gu;
   void* h = base + L.h;
-  void* d = base + L.d;
-  GenMv e{};
-  e.act = x; e.act_dt = c.x_dtype; e.act_round = T; e.act_rows = N; e.K = H;
-  e.row_expert = ridx; e.row_div = ks; e.rows = mc; e.n_out = 2 * I;
-  e.bits = c.bits; e.gs = c.group_size; e.sb_dt = c.expert_dtype; e.dense_dt = c.expert_dtype;
-  if (c.experts_packed) {
-    e.packed = static_cast<const uint32_t*>(wts->gu); e.scale = wts->gu_scale; e.bias = wts->gu_bias;
-  } else {
-    e.dense = wts->gu;
-  }
-  e.out = gu; e.out_dt = T; e.ld_out = 2 * I;
-  if ((rc = gen_matvec(e, st))) return rc;
-  const int64_t hn = mc * I;
-  gen_glu_kernel<<<dim3(static_cast<unsigned>((hn + 255) / 256)), 256, 0, st>>>(
-      gu, h, mc, I, T, c.act, c.act_alpha, c.act_limit);
-  if ((rc = check_launch("general glu"))) return rc;
-  GenMv dn = e;
-  dn.act = h; dn.act_dt = T; dn.act_round = T; dn.act_rows = mc; dn.K = I; dn.row_div = 1;
-  dn.n_out = H; dn.out = d; dn.ld_out = H;
-  if (c.experts_packed) {
-    dn.packed = static_cast<const uint32_t*>(wts->dn); dn.scale = wts->dn_scale; dn.bias = wts->dn_bias;
-  } else {
-    dn.dense = wts->dn;
-  }
-  if ((rc = gen_matvec(dn, st))) return rc;
+  const int bits = c.experts_packed ? c.bits : 0;
+  auto expert_w = [&](const void* p, const void* scale, const void* bias, int K) {
+    GenW w = dense_w(bits ? nullptr : p, c.expert_dtype, K);
+    if (bits) {
+      w.packed = static_cast<const uint32_t*>(p); w.scale = scale; w.bias = bias; w.sb_dt = c.expert_dtype;
+      w.gshift = (c.group_size == 32) ? 5 : (c.group_size == 64) ? 6 : 7;
+    }
+    return w;
+  };
+  GenGu e{};
+  e.act = x; e.act_dt = c.x_dtype; e.act_round = T; e.row_expert = ridx; e.row_div = ks; e.rows = mc;
+  e.n = I; e.n2 = 2 * I; e.up = I;
+  e.w = e.w_up = expert_w(wts->gu, wts->gu_scale, wts->gu_bias, H);
+  e.h = h; e.dt = T; e.glu = c.act; e.alpha = c.act_alpha; e.limit = c.act_limit;
+  if ((rc = gen_gate_up(e, bits, st))) return rc;
 
   // shared expert in its weights' dtype S
   void* so = nullptr;
   if (shared) {
     const int S = c.shared_dtype;
-    void* sgu = base + L.sgu;
     void* sh = base + L.sh;
     so = base + L.so;
-    GenMv s{};
-    s.act = x; s.act_dt = c.x_dtype; s.act_round = S; s.act_rows = N; s.K = H; s.row_div = 1;
-    s.rows = N; s.n_out = Is; s.dense = wts->sh_gate; s.dense_dt = S; s.out = sgu; s.out_dt = S;
-    s.ld_out = 2 * Is;
-    if ((rc = gen_matvec(s, st))) return rc;
-    s.dense = wts->sh_up; s.col0 = Is;
-    if ((rc = gen_matvec(s, st))) return rc;
-    const int64_t sn = N * Is;
-    gen_glu_kernel<<<dim3(static_cast<unsigned>((sn + 255) / 256)), 256, 0, st>>>(
-        sgu, sh, N, Is, S, c.act, c.act_alpha, c.act_limit);
-    if ((rc = check_launch("general shared glu"))) return rc;
+    GenGu s{};
+    s.act = x; s.act_dt = c.x_dtype; s.act_round = S; s.row_div = 1; s.rows = N; s.n = s.n2 = Is;
+    s.w = dense_w(wts->sh_gate, S, H);
+    s.w_up = dense_w(wts->sh_up, S, H);
+    s.h = sh; s.dt = S; s.glu = c.act; s.alpha = c.act_alpha; s.limit = c.act_limit;
+    if ((rc = gen_gate_up(s, 0, st))) return rc;
     GenMv sd{};
-    sd.act = sh; sd.act_dt = S; sd.act_round = S; sd.act_rows = N; sd.K = Is; sd.row_div = 1;
-    sd.rows = N; sd.n_out = H; sd.dense = wts->sh_down; sd.dense_dt = S; sd.out = so; sd.out_dt = S;
-    sd.ld_out = H;
+    sd.act = sh; sd.act_dt = S; sd.act_round = S; sd.rows = N; sd.n_out = H;
+    sd.w = dense_w(wts->sh_down, S, Is);
+    sd.out = so; sd.out_dt = S; sd.ld_out = H;
     if ((rc = gen_matvec(sd, st))) return rc;
   }
-  const int64_t yn = N * H;
-  gen_combine_kernel<<<dim3(static_cast<unsigned>((yn + 255) / 256)), 256, 0, st>>>(
-      d, T, rw, n, ks, H, so, c.shared_dtype, has_sg ? sg : nullptr, y, c.x_dtype);
-  return check_launch("general combine");
+  // routed down, weighted combine, gated shared expert and the cast to x's dtype
+  GenDn dn{};
+  dn.h = h; dn.dt = T; dn.idx = ridx; dn.wt = rw; dn.N = N; dn.k = ks; dn.H = H;
+  dn.w = expert_w(wts->dn, wts->dn_scale, wts->dn_bias, I);
+  dn.sh = so; dn.sh_dt = c.shared_dtype; dn.sg = has_sg ? sg : nullptr;
+  dn.y = y; dn.y_dt = c.x_dtype;
+  return gen_down_combine(dn, bits, st);
 }
