@@ -296,12 +296,13 @@ int validate_routing(int N, int H, int E, int k, int scoring, int n_group, int t
 // A fork event records the caller's stream at entry, `xready` returns the fp16 copy of x, `perm`
 // publishes the permute to the auxiliary stream, and the caller's stream waits on `join` right
 // before the combine: the cold experts' gate_up and down and the hot experts' are two chains over
-// disjoint rows of h and d, with no event between them (each wait costs the stream about 6 us). The mutex is held
+// disjoint rows of h and d, with no event between them (each wait costs the stream about 6 us), but for
+// the cold down of large layers (`hot`). The mutex is held
 // from the fork record until the join wait is enqueued, so concurrent calls on different streams
 // cannot exchange the events.
 struct AuxStream {
   hipStream_t s = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr, perm = nullptr, xready = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr, perm = nullptr, hot = nullptr, xready = nullptr;
 };
 static std::mutex g_aux_mu;
 constexpr int64_t kFuseSharedMaxTokens = 64;
@@ -354,6 +355,7 @@ static int aux_stream(hipStream_t caller, AuxStream** out) {
     if (err == hipSuccess) err = hipEventCreateWithFlags(&a.fork, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&a.join, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&a.perm, hipEventDisableTiming);
+    if (err == hipSuccess) err = hipEventCreateWithFlags(&a.hot, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&a.xready, hipEventDisableTiming);
     if (cur != dev) (void)hipSetDevice(cur);
     if (err != hipSuccess) {
@@ -373,10 +375,12 @@ static bool large_ok(const qmoe_config_t& c, int64_t N) { return N > 256 && c.hi
 // up to 256 tokens (outputs that do not depend on the batch), above that qmm_dense_kernel's 64 x 64
 // tiles, which fill the chip with small products; the large kernel's 128 x 256 tiles from the sizes
 // where they fill it too and their fewer bytes from L2 win. Whole layers, us, 64 x 64 against 128 x
-// 256 tiles: c1 391 tokens 168 / 249, c2 512 (AWQ) 887 / 946, c2 1000 960 / 991, c3 300 1285 / 1356;
-// c2 2000 1200 / 1174, c2 4096 1901 / 1850.
-constexpr double kDenseLargeMacs = 4e9;
+// 256 tiles for all three products: c2 512 tokens (AWQ) 887 / 946, c2 1000 960 / 991, c3 300 1285 / 1356,
+// c1 2048 297 / 310; c2 2000 1200 / 1174, c2 4096 1901 / 1850.
+constexpr double kDenseLargeMacs = 8e9;
 constexpr int64_t kDenseLargeTokens = 1536;
+// Weights of one projection of all experts from which the hybrid regime runs its chains in phases.
+constexpr double kPhasedLayerWeights = 1e9;
 static int dense_regime(const qmoe_config_t& c, int64_t N, int64_t rows, int64_t K) {
   if (N <= 256) return QMOE_REGIME_SMALL;
   return large_ok(c, N) && N > kDenseLargeTokens && static_cast<double>(N) * rows * K >= kDenseLargeMacs
@@ -738,7 +742,8 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
   // 128-row tile's weight dequant; under skewed routing most experts are that small while a few
   // carry thousands of rows.
   const bool hybrid = (regime == QMOE_REGIME_LARGE);
-  const int split = hybrid_split_rows(mc, c.n_experts);
+  const bool few = few_hot(mc, c.n_experts, c.inter, c.hidden);
+  const int split = few ? 32 : kHybridSplitRows;
   int32_t* tile_map_big = reinterpret_cast<int32_t*>(base + L.tile_map_big);
   const int64_t bound_small = mtile_upper_bound(mc, c.n_experts, kSmallMTile);
   const int64_t cold_bound =
@@ -1007,7 +1012,7 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
   if (hybrid && aux) {
     rc = link(aux->perm, stream, aux->s, "permute to auxiliary stream");
     if (rc) return rc;
-    (few_hot(mc, c.n_experts) ? hstream : cstream) = aux->s;
+    (few ? hstream : cstream) = aux->s;
   }
   // routed grouped matmul over the permuted rows of one class of experts: all of them on the small
   // kernel, or (hybrid) the cold ones there over their 16-row tiles and the hot ones on the large
@@ -1106,7 +1111,7 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     a.out = d; a.ld_out = c.hidden;
     if (cls == kHotExperts && f16_h) {
       const int r = launch_act_to_f16(h, mc, c.inter, h16, h_sinv, hstream,
-                                      reinterpret_cast<const int4*>(tile_map_big), hot_bound);
+                                      HotRows{sorted, idx, counts, split});
       if (r) return r;
     }
     if (!mixed) return routed(a, dfmt, EPI_BF16, h16, h_sinv, cls);
@@ -1120,13 +1125,18 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     return 0;
   };
   if (hybrid) {
-    // two chains, no event between them; enqueued in turn so that neither stream waits for the host
+    // two chains, enqueued in turn so that neither stream waits for the host
     if (f16_acts && aux && hstream == stream) {   // the fp16 copy of x, made on the auxiliary stream at the fork
       const hipError_t err = hipStreamWaitEvent(stream, aux->xready, 0);
       if (err != hipSuccess) return fail(std::string("forward: x16 wait: ") + hipGetErrorString(err));
     }
     rc = gate_up(kColdExperts);
     if (!rc) rc = gate_up(kHotExperts);
+    // In large layers the cold down waits for the hot gate_up, beside which it would take compute units
+    // from the longer chain (c2 1000 tokens 890 -> 878 us per layer, 2000 tokens 1168 -> 1155); in small
+    // ones that costs more than it gives (c1 4096 skewed tokens 519 -> 536).
+    if (!rc && cstream != stream && static_cast<double>(c.n_experts) * c.inter * c.hidden >= kPhasedLayerWeights)
+      rc = link(aux->hot, stream, aux->s, "hot gate_up");
     if (!rc) rc = down(kColdExperts);
     if (!rc) rc = down(kHotExperts);
     if (rc) return rc;

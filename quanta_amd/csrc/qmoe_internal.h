@@ -314,6 +314,8 @@ constexpr int kRegimeDense = 3;
 int launch_qmm(const QmmArgs& a, int fmt, int epi, int regime, int64_t mtile_bound,
                hipStream_t stream);
 int launch_dense(const QmmArgs& a, int fmt, int epi, hipStream_t stream);   // (dense.hip)
+// The large regime's launches (prefill.hip); launch_qmm has checked the arguments.
+int launch_large(const QmmArgs& a, int fmt, int epi, int64_t mtiles, hipStream_t stream);
 // Chunk count of the small-regime bf16 products over K: ~8 32-deep steps per chunk, one
 // wavefront per chunk, chunk sums added in chunk order.
 inline int bf16_chunks(int K) {
@@ -342,10 +344,16 @@ int launch_combine_shared(const uint16_t* d, const int32_t* inv, const float* w,
 int launch_expand_int8(const uint32_t* codes, const uint16_t* sb, int64_t rows, int K,
                        uint16_t* out, hipStream_t stream);
 // act [rows][K] bf16 -> act16 fp16 with a per-row power-of-two scale (exact for bf16 values
-// within 2^28 of the row's largest magnitude); row_sinv[r] = the inverse scale. With tiles (n_tiles
-// m-tile descriptors of at most kLargeMTile rows), only the rows of those tiles.
+// within 2^28 of the row's largest magnitude); row_sinv[r] = the inverse scale. With hot.sorted, only
+// the sorted rows whose expert (idx of the row's slot) has more than hot.split rows.
+struct HotRows {
+  const int32_t* sorted;
+  const int32_t* idx;
+  const int32_t* counts;
+  int split;
+};
 int launch_act_to_f16(const uint16_t* act, int64_t rows, int K, uint16_t* act16, float* row_sinv,
-                      hipStream_t stream, const int4* tiles = nullptr, int64_t n_tiles = 0);
+                      hipStream_t stream, const HotRows& hot = HotRows{});
 inline size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 inline size_t act16_ws_bytes(int64_t rows, int K) {
   return align256(static_cast<size_t>(rows) * K * 2) + align256(static_cast<size_t>(rows) * 4);
@@ -418,15 +426,19 @@ constexpr int kSyncStride = 64;
 
 constexpr int kSmallMTile = 16;
 constexpr int kLargeMTile = 128;
-// Large-M (prefill) regime: experts routed more rows than this use 128-row tiles on the large
+constexpr int kHybridSplitRows = 16;
+// Large-M (prefill) regime: experts routed more rows than the split use 128-row tiles on the large
 // kernel, the others 16-row tiles on the small kernel. Experts of 17 to 32 rows are cheaper as two
-// 16-row tiles (the second one's weights come from L2) while there are few of them, up to about 14
-// rows per expert on average: the large kernel's chain of a few latency-bound workgroups then
-// outlasts the cold experts' (c1 391 tokens 207 us per layer against 220, c2 600 skewed 699 / 724);
-// from 18 rows on they are most of the experts and the large kernel streams them once (c2 1000
-// tokens 982 / 1331).
-inline bool few_hot(int64_t mc, int64_t n_experts) { return mc <= 14 * n_experts; }
-inline int hybrid_split_rows(int64_t mc, int64_t n_experts) { return few_hot(mc, n_experts) ? 32 : 16; }
+// 16-row tiles while there are few of them, up to about 14 rows per expert on average: the large
+// kernel's chain of a few latency-bound workgroups then outlasts the cold experts'. From 18 rows on
+// they are most of the experts and the large kernel streams them once. The second tile's weights must
+// still come from L2: above 8 M weights per projection they are read from HBM again and the large
+// kernel's chain is short beside the cold one. Whole layers, us, 32 against 16 rows: c1 391 tokens
+// 171 / 196, c2 500 754 / 781, 128 experts of 3072 x 1536 at 400 tokens 295 / 304, c2 600 skewed 661 /
+// 711; c2 1000 1331 / 982; c3 376 1428 / 1345, c3 352 int6 2136 / 1979.
+inline bool few_hot(int64_t mc, int64_t n_experts, int64_t inter, int64_t hidden) {
+  return mc <= 14 * n_experts && inter * hidden <= (int64_t(1) << 23);
+}
 // Which experts a launch of the routed products covers: all (one regime), or the hybrid regime's
 // cold or hot ones.
 enum ExpertClass { kAllExperts = 0, kColdExperts = 1, kHotExperts = 2 };
