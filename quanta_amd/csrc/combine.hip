@@ -383,8 +383,10 @@ constexpr int64_t kDenseLargeTokens = 1536;
 constexpr double kPhasedLayerWeights = 1e9;
 static int dense_regime(const qmoe_config_t& c, int64_t N, int64_t rows, int64_t K) {
   if (N <= 256) return QMOE_REGIME_SMALL;
-  return large_ok(c, N) && N > kDenseLargeTokens && static_cast<double>(N) * rows * K >= kDenseLargeMacs
-             ? QMOE_REGIME_LARGE : kRegimeDense;
+  if (large_ok(c, N) && N > kDenseLargeTokens && static_cast<double>(N) * rows * K >= kDenseLargeMacs)
+    return QMOE_REGIME_LARGE;
+  // (qmm_dense_kernel addresses its activations with 32-bit byte offsets)
+  return N * K <= kDenseMaxActs ? kRegimeDense : QMOE_REGIME_SMALL;
 }
 static int shared_gu_regime(const qmoe_config_t& c, int64_t N) {
   return dense_regime(c, N, 2 * static_cast<int64_t>(c.shared_inter), c.hidden);

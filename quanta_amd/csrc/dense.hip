@@ -204,7 +204,7 @@ int launch_dense(const QmmArgs& a, int fmt, int epi, hipStream_t stream) {
     return fail("qmm(dense): one dense bf16 or int8 segment");
   if (a.K % 64 || a.n_rows % kDmTile || (fmt == FMT_INT8 && !a.sb))
     return fail("qmm(dense): K % 64 == 0 and weight rows % 64 == 0 required (int8: scale/bias)");
-  if (a.dense_rows * a.K > (int64_t(1) << 31) - 64) return fail("qmm(dense): activations beyond 4 GiB");
+  if (a.dense_rows * a.K > kDenseMaxActs) return fail("qmm(dense): activations beyond 4 GiB");
 #define QMOE_DENSE(F)                                                          \
   (epi == EPI_SWIGLU ? launch_dense_e<F, EPI_SWIGLU>(a, stream)                \
    : epi == EPI_BF16 ? launch_dense_e<F, EPI_BF16>(a, stream)                  \

@@ -311,6 +311,7 @@ enum { EPI_SWIGLU = 0, EPI_BF16 = 1, EPI_F32 = 2 };
 // regime: QMOE_REGIME_SMALL, QMOE_REGIME_LARGE, or kRegimeDense (dense products of batches above
 // the decode sizes, qmm_dense_kernel; mtile_bound unused).
 constexpr int kRegimeDense = 3;
+constexpr int64_t kDenseMaxActs = (int64_t(1) << 31) - 64;   // its activations, elements (4 GiB)
 int launch_qmm(const QmmArgs& a, int fmt, int epi, int regime, int64_t mtile_bound,
                hipStream_t stream);
 int launch_dense(const QmmArgs& a, int fmt, int epi, hipStream_t stream);   // (dense.hip)
