@@ -99,7 +99,7 @@ COPY_BYTES = 2 << 30          # the 2 GiB device copy of the `--only kernel` run
 
 def kernel_key(workload, regime_small):
     """Counter-CSV kernel name prefix of the routed gate_up+SwiGLU launch."""
-    return "qmm_small_kernel<0, 0," if regime_small else "qmm_wide_kernel<0>"
+    return "qmm_small_kernel<0, 0," if regime_small else "prefill_kernel<0, 0, 2>"
 
 
 def write_traffic(fetch_dir, write_dir, workload="c2-decode-N32", regime_small=True, reps=8):
@@ -353,7 +353,7 @@ def main():
         per_expert = 2 * I * H * 9 // 16                   # int4 codes + bf16 scale/bias per 64
         kbytes = u_k * per_expert + N * H * 2 + N * k * I * 2
         kern = dict(name="qmm_small_kernel<int4,swiglu,W,CPW,JPW>" if regime == L.REGIME_SMALL
-                    else "act_to_f16 + qmm_wide_kernel<swiglu>", us=kms * 1e3, bytes=kbytes,
+                    else "act_to_f16 + prefill_kernel<int4,swiglu,2>", us=kms * 1e3, bytes=kbytes,
                     U=u_k, mfma=regime == L.REGIME_LARGE, flops=2 * N * k * 2 * I * H)
         log(f"gate_up kernel: {kms * 1e3:.1f} us, {kbytes / kms / 1e6:.0f} GB/s")
 
