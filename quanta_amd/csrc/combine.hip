@@ -910,10 +910,13 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     // are padding for the large kernel's 256-row tiles)
     const int live_rows = (c.n_experts + has_sg + 15) / 16 * 16;
     a.act = x; a.act_rows = N; a.slot_div = 1; a.dense_rows = N; a.n_experts = 1;
-    const int rreg = dense_regime(c, N, live_rows, c.hidden);
+    // Above the decode sizes a logit is one sum over all of K in k order, whichever of two kernels forms it
+    // (the large kernel, or router_logits_kernel below its sizes), as the large regime's always was: a split
+    // of K moves tokens across near-ties to other experts. Hidden sizes off 256 keep the decode kernel.
+    const bool rlarge = dense_regime(c, N, live_rows, c.hidden) == QMOE_REGIME_LARGE;
+    const bool rmid = large_ok(c, N) && !rlarge;
     a.K = c.hidden;
-    a.n_rows = (rreg == QMOE_REGIME_SMALL) ? std::min(live_rows, c.router_rows)
-               : (rreg == kRegimeDense) ? (live_rows + 63) / 64 * 64 : c.router_rows;
+    a.n_rows = rlarge ? c.router_rows : rmid ? (live_rows + 63) / 64 * 64 : std::min(live_rows, c.router_rows);
     a.codes = wts->router_w; a.out = logits; a.ld_out = ld;
     if (fuse_norm) {   // both products read the raw rows and normalise them; the router writes xn
       a.act = x_in; a.norm_w = norm_w; a.norm_eps = norm_eps; a.norm_out = xn;
@@ -921,8 +924,8 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     }
     // (large regime: 64-token m-tiles, so the few row blocks of the router still give twice
     // as many workgroups)
-    const int rt = (rreg == QMOE_REGIME_LARGE) ? 64 : kSmallMTile;
-    if (rreg == QMOE_REGIME_LARGE) a.dense_mtile = rt;
+    const int rt = rlarge ? 64 : kSmallMTile;
+    if (rlarge) a.dense_mtile = rt;
     if (use_flow) {
       a.zero_words = sync;
       a.n_zero = static_cast<int>(L.sync_words / kSyncStride);
@@ -946,8 +949,10 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
       const bool split = use_flow && decode_flow_split_shared(c.hidden, c.inter, c.shared_inter);
       if (split) sgu.ld_out = 2 * c.shared_inter;
       rc = launch_qmm_pair_bf16(a, sgu, stream, sfmt, split);
+    } else if (rmid) {
+      rc = launch_router_logits(a, stream);
     } else {
-      rc = launch_qmm(a, FMT_BF16, EPI_F32, rreg, (N + rt - 1) / rt, stream);
+      rc = launch_qmm(a, FMT_BF16, EPI_F32, rlarge ? QMOE_REGIME_LARGE : QMOE_REGIME_SMALL, (N + rt - 1) / rt, stream);
     }
   }
   if (rc) return rc;

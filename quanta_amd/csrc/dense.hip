@@ -1,8 +1,8 @@
-// Dense products of batches above the decode sizes: the router logits and the shared expert's gate_up
-// and down projections over more than 256 tokens (tiled bf16 or int8 weights).
+// Dense products of batches above the decode sizes: the shared expert's gate_up and down projections over
+// more than 256 tokens (tiled bf16 or int8 weights). The router's logits have a kernel of their own
+// (prefill.hip): their sums must not depend on how K is cut.
 //
-// Reference: the router matmul src/quanta/qwen35/moe.py:47; the shared expert's matmuls
-// src/quanta/qwen35/moe.py:145-151.
+// Reference: the shared expert's matmuls src/quanta/qwen35/moe.py:145-151.
 //
 // Each wavefront holds a 64-token x 64-weight-row tile (SwiGLU: 32 gate + 32 up rows; 4 x 4 16x16
 // blocks) and reads its fragments straight from L2 in 64-deep stages, two in registers. KS of the
@@ -200,15 +200,13 @@ static int launch_dense_e(const QmmArgs& a, hipStream_t stream) {
 }
 
 int launch_dense(const QmmArgs& a, int fmt, int epi, hipStream_t stream) {
-  if (!fmt_dense(fmt) || a.offsets || a.tile_map || a.dense_rows <= 0 || a.act_stride || a.norm_w)
-    return fail("qmm(dense): one dense bf16 or int8 segment");
+  if (!fmt_dense(fmt) || epi == EPI_F32 || a.offsets || a.tile_map || a.dense_rows <= 0 || a.act_stride || a.norm_w)
+    return fail("qmm(dense): one dense bf16 or int8 segment, bf16 out");
   if (a.K % 64 || a.n_rows % kDmTile || (fmt == FMT_INT8 && !a.sb))
     return fail("qmm(dense): K % 64 == 0 and weight rows % 64 == 0 required (int8: scale/bias)");
   if (a.dense_rows * a.K > kDenseMaxActs) return fail("qmm(dense): activations beyond 4 GiB");
-#define QMOE_DENSE(F)                                                          \
-  (epi == EPI_SWIGLU ? launch_dense_e<F, EPI_SWIGLU>(a, stream)                \
-   : epi == EPI_BF16 ? launch_dense_e<F, EPI_BF16>(a, stream)                  \
-                     : launch_dense_e<F, EPI_F32>(a, stream))
+#define QMOE_DENSE(F) \
+  (epi == EPI_SWIGLU ? launch_dense_e<F, EPI_SWIGLU>(a, stream) : launch_dense_e<F, EPI_BF16>(a, stream))
   const int rc = (fmt == FMT_INT8) ? QMOE_DENSE(FMT_INT8) : QMOE_DENSE(FMT_BF16);
 #undef QMOE_DENSE
   return rc ? rc : check_launch("qmm(dense)");

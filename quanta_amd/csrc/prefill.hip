@@ -1,5 +1,5 @@
 // Large-M ("prefill") products over 128-position m-tiles, for gfx950: the routed experts' gate_up and down
-// above the decode sizes, and large dense bf16 products (router, shared expert).
+// above the decode sizes, router logits there, and large dense bf16 products (router, shared expert).
 //
 // Reference: mx.gather_qmm over sorted rows src/quanta/dsv4/moe.py:114-124 and
 // src/quanta/qwen35/moe.py:117-123; SwiGLU src/quanta/qwen35/moe.py:59-63; bf16 experts
@@ -617,6 +617,110 @@ __global__ void __launch_bounds__(kPfThreads) qmm_large_kernel(QmmArgs a) {
       }
     }
   }
+}
+
+// ============================================================================ router logits
+// Logits of batches above the decode sizes, short of those that fill the chip with qmm_large_kernel's tiles:
+// 16 MB tokens x 64 weight rows per workgroup, a 128-deep k superblock per iteration, two 16x16 blocks per
+// wavefront (weight tile w % 4, m-blocks 2 (w / 4) and the next), tokens and weights through an LDS ring
+// ([16-row block][step][64 lanes] x 16 B).
+//
+// Every logit is one accumulator over all of K in k order, which is qmm_large_kernel's sum: the expert ids of a
+// prompt depend on neither the kernel that a batch size takes nor K's split over wavefronts, whose sums
+// differ by up to 8e-6 at c2 and move a token across a tie of its last expert now and then.
+//
+// What bounds it is the latency of the loads, K / 128 dependent rounds: the ring keeps them NS - 1 superblocks
+// ahead.
+template <int MB>
+struct RouterCfg {
+  static constexpr int WAVES = 2 * MB;                       // MB = 2 or 4
+  static constexpr int SLOT = (MB + 4) * 4096;               // one superblock: MB token blocks, 4 weight tiles
+  static constexpr int NS = (MB == 2) ? 6 : 4;
+  static constexpr int LOADS = 2 + 16 / WAVES;               // per wavefront and superblock
+  static constexpr size_t LDS = static_cast<size_t>(NS) * SLOT;   // 144 or 128 KiB
+};
+
+template <int MB>
+__global__ void __launch_bounds__(64 * RouterCfg<MB>::WAVES) router_logits_kernel(QmmArgs a, int n_tok, int n_rb, int n_wg) {
+  using C = RouterCfg<MB>;
+  extern __shared__ u32x4 lds[];
+  const char* lds_c = reinterpret_cast<const char*>(lds);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  // (each XCD takes a run of tiles, a token block's weight blocks together: its L2 reads its share of x once)
+  const int per = (n_wg + 7) / 8;
+  const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (static_cast<int>(blockIdx.x >> 3) >= per || id >= n_wg) return;
+  const int tb = id / n_rb, rb = id % n_rb;
+  const int rows = static_cast<int>(a.dense_rows);
+  const int nsb = a.K / 128;
+  // loads: two steps of token block ab, and 16 / WAVES steps of weight tile w % 4. Tokens past the end read row 0
+  // (never stored).
+  const int ab = (MB == 2) ? wave >> 1 : wave & 3, as = 2 * ((MB == 2) ? wave & 1 : wave >> 2);
+  const int ws = (16 / C::WAVES) * (wave >> 2);
+  const int t = 16 * MB * tb + 16 * ab + (lane & 15);
+  const char* xp = reinterpret_cast<const char*>(a.act + (t < rows ? t : 0) * static_cast<int64_t>(a.K)) + 16 * (lane >> 4);
+  const char* wp = static_cast<const char*>(a.codes) + (4 * rb + (wave & 3)) * static_cast<int64_t>(a.K / 32) * 1024;
+  const uint32_t lds_base = lds_offset(lds);
+  auto issue = [&](int p) __attribute__((always_inline)) {
+    const uint32_t dst = lds_base + p % C::NS * C::SLOT;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) dma16(xp + 256 * p + 64 * (as + j), dst + (4 * ab + as + j) * 1024);
+#pragma unroll
+    for (int j = 0; j < 16 / C::WAVES; ++j)
+      dma16s(wp + (4 * static_cast<int64_t>(p) + ws + j) * 1024, 16 * lane, dst + (4 * (MB + (wave & 3)) + ws + j) * 1024);
+  };
+  const int n0 = min(C::NS - 1, nsb);
+  for (int p = 0; p < n0; ++p) issue(p);
+  const int mb = 2 * (wave >> 2);
+  f32x4_t acc[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int p = 0; p < nsb; ++p) {
+    // this wavefront's loads of superblock p have landed (those of the NS - 2 after it may be in flight); the
+    // barrier publishes p and retires p - 1, whose slot the loads of p + NS - 1 take
+    if (p + C::NS - 2 < nsb) wait_vmcnt<(C::NS - 2) * C::LOADS>(); else wait_vmcnt<0>();
+    lg_barrier();
+    if (p + C::NS - 1 < nsb) issue(p + C::NS - 1);
+    const u32x4* sl = reinterpret_cast<const u32x4*>(lds_c + p % C::NS * C::SLOT) + lane;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const bf16x8_t B = as_bf16x8(sl[256 * (MB + (wave & 3)) + 64 * s]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] = mfma16(as_bf16x8(sl[256 * (mb + i) + 64 * s]), B, acc[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = 16 * (MB * tb + mb + i) + 4 * (lane >> 4) + j;
+      if (row < rows) store_out<EPI_F32>(a, row, 64 * rb + 16 * (wave & 3) + (lane & 15), acc[i][j], 0.f);
+    }
+}
+
+template <int MB>
+static int launch_router_k(const QmmArgs& a, hipStream_t stream) {
+  using C = RouterCfg<MB>;
+  const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(router_logits_kernel<MB>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(C::LDS));
+  if (err != hipSuccess) return fail(std::string("router logits: LDS attribute: ") + hipGetErrorString(err));
+  const int64_t n_tok = (a.dense_rows + 16 * MB - 1) / (16 * MB), n_rb = a.n_rows / 64, n_wg = n_tok * n_rb;
+  if (n_wg > (int64_t(1) << 30)) return fail("router logits: product too large for one launch");
+  router_logits_kernel<MB><<<dim3(static_cast<unsigned>((n_wg + 7) / 8 * 8)), 64 * C::WAVES, C::LDS, stream>>>(
+      a, static_cast<int>(n_tok), static_cast<int>(n_rb), static_cast<int>(n_wg));
+  return check_launch("router logits");
+}
+
+int launch_router_logits(const QmmArgs& a, hipStream_t stream) {
+  if (a.offsets || a.tile_map || a.dense_rows <= 0 || a.dense_rows > (int64_t(1) << 30) || a.act_stride || a.norm_w)
+    return fail("router logits: one dense bf16 segment");
+  if (a.K <= 0 || a.K % 128 || a.n_rows <= 0 || a.n_rows % 64)
+    return fail("router logits: K % 128 == 0 and weight rows % 64 == 0 required");
+  // 32-token tiles while they are at most a workgroup per CU (us, 32 against 64 tokens: c2 1000 tokens 16 / 22,
+  // c1 391 10 / 12, c1 2048 11 / 13, 7168 x 256 700 17 / 21), 64-token ones above, where a second wave of the
+  // smaller ones would read a third more (c2 1536 30 / 23).
+  const bool two = (a.dense_rows + 31) / 32 * (a.n_rows / 64) <= 256;
+  return two ? launch_router_k<2>(a, stream) : launch_router_k<4>(a, stream);
 }
 
 // ============================================================================ launcher

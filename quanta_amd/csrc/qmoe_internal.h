@@ -308,8 +308,8 @@ __device__ __forceinline__ u32x4 dense_bf16(const DenseFrag<FMT>& f) {
 }
 enum { EPI_SWIGLU = 0, EPI_BF16 = 1, EPI_F32 = 2 };
 
-// regime: QMOE_REGIME_SMALL, QMOE_REGIME_LARGE, or kRegimeDense (dense products of batches above
-// the decode sizes, qmm_dense_kernel; mtile_bound unused).
+// regime: QMOE_REGIME_SMALL, QMOE_REGIME_LARGE, or kRegimeDense (the shared expert's products in batches
+// above the decode sizes, qmm_dense_kernel; mtile_bound unused).
 constexpr int kRegimeDense = 3;
 constexpr int64_t kDenseMaxActs = (int64_t(1) << 31) - 64;   // its activations, elements (4 GiB)
 int launch_qmm(const QmmArgs& a, int fmt, int epi, int regime, int64_t mtile_bound,
@@ -317,6 +317,8 @@ int launch_qmm(const QmmArgs& a, int fmt, int epi, int regime, int64_t mtile_bou
 int launch_dense(const QmmArgs& a, int fmt, int epi, hipStream_t stream);   // (dense.hip)
 // The large regime's launches (prefill.hip); launch_qmm has checked the arguments.
 int launch_large(const QmmArgs& a, int fmt, int epi, int64_t mtiles, hipStream_t stream);
+// Dense bf16 x bf16 -> fp32 (router logits), each sum in the large regime's order (prefill.hip).
+int launch_router_logits(const QmmArgs& a, hipStream_t stream);
 // Chunk count of the small-regime bf16 products over K: ~8 32-deep steps per chunk, one
 // wavefront per chunk, chunk sums added in chunk order.
 inline int bf16_chunks(int K) {

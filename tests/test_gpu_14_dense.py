@@ -1,6 +1,6 @@
-"""GPU tier: the dense products of batches above the decode sizes (dense.hip `qmm_dense_kernel`: router
-logits and the shared expert over 64-token x 64-row tiles) and the two-chain hybrid regime around
-them, against the oracle.
+"""GPU tier: the dense products of batches above the decode sizes (dense.hip `qmm_dense_kernel`: the shared
+expert over 64-token x 64-row tiles; prefill.hip `router_logits_kernel`) and the two-chain hybrid
+regime around them, against the oracle.
 
 The shapes sit where the kernel's tiling can go wrong: hidden and shared sizes for each number of
 wavefronts that cut K (1, 2, 4 and 8, with stages that do not divide evenly), weight-row blocks that
@@ -16,8 +16,9 @@ import pytest
 import torch
 
 from oracle import moe as om
-from quanta_amd import synth
-from quanta_amd.moe import qwen35_moe
+from quanta_amd import _lib as L
+from quanta_amd import ops, synth
+from quanta_amd.moe import prepare, qwen35_moe
 from quanta_amd.quant import quantize_affine
 from tests._util import assert_close, f64, oracle_params_from_torch
 
@@ -43,6 +44,29 @@ def test_dense_products_vs_oracle(gpu, N, H, Is, E, bits):
     y = qwen35_moe(x[None], p, s.cfg)[0]
     _, it = om.moe_forward(f64(x), oracle_params_from_torch(p), k=2, inter=128)
     assert_close(f64(y), it["y_exact"], f"dense N={N} H={H} Is={Is} E={E} int{bits}")
+
+
+@pytest.mark.parametrize("N,H,E", [(257, 256, 16), (300, 640, 40), (513, 512, 255), (700, 2048, 256), (1000, 768, 64),
+                                   (1023, 4096, 512), (1537, 4096, 512)])
+def test_router_logits_keep_their_order(gpu, N, H, E):
+    """Router logits above the decode sizes are one fp32 sum over all of K in k order, bit for bit the large
+    kernel's (hidden sizes off 256: the decode kernel's), so that a prompt's expert ids do not depend on
+    the kernel its size takes. 32- and 64-token tiles, last tiles partly filled, fewer superblocks than the
+    ring holds, rows with and without the shared gate's past the last block of 16. (The workspace starts with
+    the logits.)"""
+    s = synth.scaled_spec("c1", hidden_size=H, num_experts=E, num_experts_per_tok=2,
+                          moe_intermediate_size=128, shared_expert_intermediate_size=128)
+    p = synth.make_layer(s, device=gpu, seed=N)
+    pr = prepare(p, s.cfg, topk=2)
+    rows = pr.cfg.router_rows
+    x = synth.make_inputs(s, N, device=gpu, seed=N)
+    ws = torch.zeros(ops.forward_workspace(pr.cfg, N), dtype=torch.uint8, device=gpu)
+    ops.forward(pr.cfg, pr.weights, x, ws=ws)
+    got = ws[: N * rows * 4].view(torch.float32).view(N, rows)[:, : E + 1]
+    want = ops.grouped_qmm(x, K=H, n_rows=rows, weight_format=L.FMT_BF16, codes=pr.router_tiled, sb=None,
+                           out_rows=N, epilogue=L.EPI_F32, dense_rows=N,
+                           regime=L.REGIME_LARGE if H % 256 == 0 else L.REGIME_SMALL)[:, : E + 1]
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("E,N", [(64, 300), (32, 400), (8, 300)])
