@@ -257,7 +257,8 @@ def _matches(sig: tuple, o) -> bool:
     an int8 shared expert)."""
     kind = sig[0]
     if kind == _LEAF:
-        return sig[1]() is o and (sig[2] is None or o._version == sig[2])
+        # (a reference whose leaf is gone reads None, which is no match for a source that is None now)
+        return o is not None and sig[1]() is o and (sig[2] is None or o._version == sig[2])
     if kind == _VALUE:
         v = sig[1]
         return o is v or (type(o) is type(v) and o == v)
