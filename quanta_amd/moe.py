@@ -774,15 +774,19 @@ def _cfg_key(cfg) -> tuple:
     return _CFG_VALUES(cfg) if type(cfg) is MoEConfig else tuple(getattr(cfg, f, None) for f in _CFG_FIELDS)
 
 
-# QmoeGeneralConfig by the values it is made of (no tensors); emptied when it reaches its bound
+# QmoeGeneralConfig by the plain values it is made of; emptied when it reaches its bound
 _GENERAL_CFG: dict = {}
 _GENERAL_CFG_MAX = 256
+_PLAIN = frozenset((int, float, bool, str, type(None)))
 
 
 def _general_config(cfg, topk: int, x_dt: int, gate_dt: int, experts: tuple, shared_dt: int | None,
                     sgate_dt: int | None, has_bias: bool, dense_all: bool) -> L.QmoeGeneralConfig:
-    key = (_cfg_key(cfg), topk, x_dt, gate_dt, experts, shared_dt, sgate_dt, has_bias, dense_all)
-    c = _GENERAL_CFG.get(key)
+    values = _cfg_key(cfg)
+    # (anything else a config holds, an array or a tensor, may have no hash or change in place: read each time)
+    plain = _PLAIN.issuperset(map(type, values))
+    key = (values, topk, x_dt, gate_dt, experts, shared_dt, sgate_dt, has_bias, dense_all)
+    c = _GENERAL_CFG.get(key) if plain else None
     if c is not None:
         return c
     scoring = str(_cfg(cfg, "scoring_func", "softmax"))
@@ -803,9 +807,10 @@ def _general_config(cfg, topk: int, x_dt: int, gate_dt: int, experts: tuple, sha
     c.topk_group = int(_cfg(cfg, "topk_group", 1))
     c.routed_scale = float(_cfg(cfg, "routed_scaling_factor", 1.0))
     c.act, c.act_alpha, c.act_limit = gated_activation(cfg)
-    if len(_GENERAL_CFG) >= _GENERAL_CFG_MAX:
-        _GENERAL_CFG.clear()
-    _GENERAL_CFG[key] = c
+    if plain:
+        if len(_GENERAL_CFG) >= _GENERAL_CFG_MAX:
+            _GENERAL_CFG.clear()
+        _GENERAL_CFG[key] = c
     return c
 
 

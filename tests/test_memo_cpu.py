@@ -1,5 +1,6 @@
-"""CPU tier: the memo of resident forms (moe._memo): an entry is reused only while every source it was built
-from is the same object at the same version, and a source that goes away is a change like any other."""
+"""CPU tier: the host path of the module calls. The memo of resident forms (moe._memo): an entry is reused only
+while every source it was built from is the same object at the same version, and a source that goes away is a
+change like any other. The config struct of the reference-dtype block, and the stream query."""
 
 from __future__ import annotations
 
@@ -56,3 +57,22 @@ def test_changes_that_rebuild_and_calls_that_do_not():
     assert run([{"packed": t, "bits": 3}, (t, 1)]) == 4
     assert run([{"packed": t, "bits": 3}, [t, 1]]) == 4
     assert run([t, [t, 1]]) == 5
+
+
+@pytest.mark.parametrize("value", [lambda v: v, np.array, torch.tensor, np.float32])
+def test_general_config_values(value):
+    """The reference-dtype block's config struct: kept for plain values, read again from a config that holds an
+    array or a tensor, which may have no hash or be written in place."""
+    from types import SimpleNamespace
+
+    limit = value(7.0)
+    cfg = SimpleNamespace(hidden_size=32, num_experts=4, num_experts_per_tok=2, moe_intermediate_size=64,
+                          swiglu_limit=limit)
+    get = lambda: M._general_config(cfg, 2, 0, 0, (True, 0, 4, 32), None, None, False, False)
+    assert get().act_limit == 7.0 and get().top_k == 2
+    if isinstance(limit, (np.ndarray, torch.Tensor)):
+        limit -= 2.0
+    else:
+        cfg.swiglu_limit = value(5.0)
+    assert get().act_limit == 5.0
+    assert len(M._GENERAL_CFG) <= M._GENERAL_CFG_MAX
