@@ -19,10 +19,16 @@ def _stream(dev: torch.device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
+# (private to torch: the public query below stands in where a build has none)
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _raw_stream(t: torch.Tensor) -> int:
     """torch's current stream of the tensor's device as a raw handle, without building the Stream
     object (2 us per call)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    if _current_raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _current_raw_stream(t.get_device())
 
 
 def _p(t: torch.Tensor | None) -> ctypes.c_void_p | None:

@@ -76,3 +76,13 @@ def test_general_config_values(value):
         cfg.swiglu_limit = value(5.0)
     assert get().act_limit == 5.0
     assert len(M._GENERAL_CFG) <= M._GENERAL_CFG_MAX
+
+
+def test_raw_stream_without_the_private_query(monkeypatch):
+    from types import SimpleNamespace
+
+    from quanta_amd import ops
+
+    monkeypatch.setattr(ops, "_current_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev: SimpleNamespace(cuda_stream=(dev.type, 7)))
+    assert ops._raw_stream(torch.zeros(1)) == ("cpu", 7)
