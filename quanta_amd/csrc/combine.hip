@@ -371,28 +371,47 @@ static int aux_stream(hipStream_t caller, AuxStream** out) {
 // widths (hidden for the down projection) to be multiples of the 256-row tile.
 static bool large_ok(const qmoe_config_t& c, int64_t N) { return N > 256 && c.hidden % 256 == 0; }
 
-// Regime of a dense product (router, shared expert) of `rows` weight rows over K: the decode kernel
-// up to 256 tokens (outputs that do not depend on the batch), above that qmm_dense_kernel's 64 x 64
-// tiles, which fill the chip with small products; the large kernel's 128 x 256 tiles from the sizes
-// where they fill it too and their fewer bytes from L2 win. Whole layers, us, 64 x 64 against 128 x
-// 256 tiles for all three products: c2 512 tokens (AWQ) 887 / 946, c2 1000 960 / 991, c3 300 1285 / 1356,
-// c1 2048 297 / 310; c2 2000 1200 / 1174, c2 4096 1901 / 1850.
-constexpr double kDenseLargeMacs = 8e9;
-constexpr int64_t kDenseLargeTokens = 1536;
-// Weights of one projection of all experts from which the hybrid regime runs its chains in phases.
-constexpr double kPhasedLayerWeights = 1e9;
-static int dense_regime(const qmoe_config_t& c, int64_t N, int64_t rows, int64_t K) {
+// Regime of a shared-expert product of `rows` weight rows over K: the decode kernel up to 256 tokens (outputs
+// that do not depend on the batch), above that qmm_dense_kernel's 64 x 64 tiles, which fill the chip with
+// small products, and the large kernel's 128 x 256 tiles where about 100 of them (3e6 outputs) do as well and
+// their fewer bytes from L2 win. The gate_up runs beside the routing chain, which the large tiles hold up, so
+// it also takes 1e10 multiply-adds, or twice the outputs; the down runs beside the hot experts and is half
+// the work. Fewer than 640 tokens leave too much of the 128-token tiles empty. Whole layers, us, int8 weights
+// (bf16 alike), 64 x 64 against 128 x 256 tiles (hidden x shared intermediate at tokens):
+//   gate_up  7168 x 2048 600 1453 / 1502, 800 1531 / 1559, 1000 1695 / 1685, 1500 2079 / 2001; 4096 x 1024 1000
+//            883 / 907, 1500 990 / 1004, 2000 1151 / 1155, 3000 1392 / 1375; 2048 x 512 4096 445 / 477, 6000 618 / 601;
+//            4096 x 4096 450 265 / 278, 650 363 / 332; 7168 x 8192 500 627 / 697, 640 771 / 760, 1200 1237 / 1149;
+//            3072 x 3072 650 251 / 227; 1024 x 1024 3000 155 / 150; 5120 x 512 2000 708 / 714, 3000 945 / 886;
+//            8192 x 256 3000 470 / 514
+//   down     7168 x 2048 520 1438 / 1435, 850 1584 / 1555; 4096 x 1024 860 867 / 868, 1500 990 / 978; 2048 x 512 1024
+//            220 / 224, 1950 285 / 281; 4096 x 4096 700 350 / 364, 980 459 / 434; 3072 x 3072 1100 329 / 325;
+//            2048 x 8192 1000 387 / 437, 1600 572 / 544; 1024 x 1024 3000 155 / 161, 4000 216 / 212
+// (`alone` outputs are enough by themselves; from 3e6 on, with `macs` multiply-adds)
+constexpr int64_t kDenseLargeTokens = 640;
+static int shared_regime(const qmoe_config_t& c, int64_t N, int64_t rows, int64_t K, int64_t alone, double macs) {
   if (N <= 256) return QMOE_REGIME_SMALL;
-  if (large_ok(c, N) && N > kDenseLargeTokens && static_cast<double>(N) * rows * K >= kDenseLargeMacs)
+  const int64_t outs = N * rows;
+  if (large_ok(c, N) && N >= kDenseLargeTokens &&
+      (outs >= alone || (outs >= 3000000 && static_cast<double>(outs) * K >= macs)))
     return QMOE_REGIME_LARGE;
   // (qmm_dense_kernel addresses its activations with 32-bit byte offsets)
   return N * K <= kDenseMaxActs ? kRegimeDense : QMOE_REGIME_SMALL;
 }
+// Weights of one projection of all experts from which the hybrid regime runs its chains in phases.
+constexpr double kPhasedLayerWeights = 1e9;
 static int shared_gu_regime(const qmoe_config_t& c, int64_t N) {
-  return dense_regime(c, N, 2 * static_cast<int64_t>(c.shared_inter), c.hidden);
+  return shared_regime(c, N, 2 * static_cast<int64_t>(c.shared_inter), c.hidden, 6000000, 1e10);
 }
 static int shared_dn_regime(const qmoe_config_t& c, int64_t N) {
-  return dense_regime(c, N, c.hidden, c.shared_inter);
+  return shared_regime(c, N, c.hidden, c.shared_inter, 4000000, 2.5e10);
+}
+
+// Whether the router's logits above the decode sizes take the large kernel: beyond router_logits_kernel's one
+// 64-token tile per CU, but for a long K, which the large kernel's few tiles walk more slowly. Whole layers,
+// us, router_logits_kernel against the large kernel: c1 2048 tokens 279 / 291, 4096 457 / 443, 8192 750 / 722;
+// c2 1536 981 / 994, 2000 1114 / 1114, 3000 1333 / 1319, 4096 1594 / 1578; c3 2500 2541 / 2592, 4096 3805 / 3881.
+static bool router_large(const qmoe_config_t& c, int64_t N, int64_t rows) {
+  return large_ok(c, N) && c.hidden <= 4096 && (N + 63) / 64 * ((rows + 63) / 64) > 256;
 }
 
 // Whether a projection of an int8 shared expert is expanded to bf16 for this call: the large-M
@@ -913,7 +932,7 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     // Above the decode sizes a logit is one sum over all of K in k order, whichever of two kernels forms it
     // (the large kernel, or router_logits_kernel below its sizes), as the large regime's always was: a split
     // of K moves tokens across near-ties to other experts. Hidden sizes off 256 keep the decode kernel.
-    const bool rlarge = dense_regime(c, N, live_rows, c.hidden) == QMOE_REGIME_LARGE;
+    const bool rlarge = router_large(c, N, live_rows);
     const bool rmid = large_ok(c, N) && !rlarge;
     a.K = c.hidden;
     a.n_rows = rlarge ? c.router_rows : rmid ? (live_rows + 63) / 64 * 64 : std::min(live_rows, c.router_rows);
