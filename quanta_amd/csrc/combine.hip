@@ -504,6 +504,7 @@ static int kernel_fmt(int f) {
   return f == QMOE_FMT_INT4_G64 ? FMT_INT4 : f == QMOE_FMT_INT6_G64 ? FMT_INT6
          : f == QMOE_FMT_INT3_G64 ? FMT_INT3 : f == QMOE_FMT_INT8_G64 ? FMT_INT8 : FMT_BF16;
 }
+static int weight_bits(int kfmt) { return kfmt == FMT_INT3 ? 3 : kfmt == FMT_INT4 ? 4 : kfmt == FMT_INT6 ? 6 : 16; }
 // AWQ-scaled experts in the large regime: quantized weights (awq implies them), and gate and up
 // halves that split at a whole 256-row block (the large kernels pick the activation copy per
 // weight-row block)
@@ -763,7 +764,7 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
   // 128-row tile's weight dequant; under skewed routing most experts are that small while a few
   // carry thousands of rows.
   const bool hybrid = (regime == QMOE_REGIME_LARGE);
-  const bool few = few_hot(mc, c.n_experts, c.inter, c.hidden);
+  const bool few = few_hot(mc, c.n_experts, c.inter, c.hidden, weight_bits(mixed ? FMT_INT4 : kernel_fmt(c.expert_format)));
   const int split = few ? 32 : kHybridSplitRows;
   int32_t* tile_map_big = reinterpret_cast<int32_t*>(base + L.tile_map_big);
   const int64_t bound_small = mtile_upper_bound(mc, c.n_experts, kSmallMTile);

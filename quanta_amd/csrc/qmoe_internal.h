@@ -429,18 +429,26 @@ constexpr int kSyncStride = 64;
 
 constexpr int kSmallMTile = 16;
 constexpr int kLargeMTile = 128;
-constexpr int kHybridSplitRows = 16;
 // Large-M (prefill) regime: experts routed more rows than the split use 128-row tiles on the large
 // kernel, the others 16-row tiles on the small kernel. Experts of 17 to 32 rows are cheaper as two
-// 16-row tiles while there are few of them, up to about 14 rows per expert on average: the large
-// kernel's chain of a few latency-bound workgroups then outlasts the cold experts'. From 18 rows on
-// they are most of the experts and the large kernel streams them once. The second tile's weights must
-// still come from L2: above 8 M weights per projection they are read from HBM again and the large
-// kernel's chain is short beside the cold one. Whole layers, us, 32 against 16 rows: c1 391 tokens
-// 171 / 196, c2 500 754 / 781, 128 experts of 3072 x 1536 at 400 tokens 295 / 304, c2 600 skewed 661 /
-// 711; c2 1000 1331 / 982; c3 376 1428 / 1345, c3 352 int6 2136 / 1979.
-inline bool few_hot(int64_t mc, int64_t n_experts, int64_t inter, int64_t hidden) {
-  return mc <= 14 * n_experts && inter * hidden <= (int64_t(1) << 23);
+// 16-row tiles while there are few of them: the large kernel's chain of a few latency-bound
+// workgroups then outlasts the cold experts'. The limit in rows per expert on average falls with the
+// weight bytes, which the second tile reads again and beside which that chain is short. us per layer, 32
+// against 16 rows:
+//   to 80 MB a projection   16: 64 experts 1024 x 2048 int4 16 rows 131 / 143, 17 146 / 144; 1536 x 768 16 100 / 107;
+//                               128 experts 1024 x 512 16 113 / 114, 22 128 / 112
+//   to 160 MB               13: 256 experts 2048 x 512 (c1) int4 13 160 / 175, 14 179 / 180; int3 14.5 166 / 171;
+//                               64 experts 1024 x 2048 int6 13 134 / 147, 15 153 / 150
+//   above                   11: c1 int6 11 204 / 212, 12 214 / 211; c1 bf16 11 361 / 388, 12.5 378 / 378; c2 int4 11
+//                               789 / 810, 12.5 833 / 807, 14 913 / 830; c2 int6 10.5 1186 / 1197, 14 1411 / 1236;
+//                               512 experts 2048 x 512 11 261 / 270, 12 272 / 271; 128 of 4096 x 2048 int4 12 419 /
+//                               439, 14 459 / 431, int6 11 612 / 626, 12 647 / 638
+// The second tile's weights must still come from L2: above 8 M weights per projection they are read from
+// HBM again (c3 376 tokens 1428 / 1345, c3 352 int6 2136 / 1979).
+constexpr int kHybridSplitRows = 16;
+inline bool few_hot(int64_t mc, int64_t n_experts, int64_t inter, int64_t hidden, int bits) {
+  const int64_t mb = n_experts * inter * hidden * bits / 8 / 1000000;
+  return mc <= (mb <= 80 ? 16 : mb <= 160 ? 13 : 11) * n_experts && inter * hidden <= (int64_t(1) << 23);
 }
 // Which experts a launch of the routed products covers: all (one regime), or the hybrid regime's
 // cold or hot ones.
