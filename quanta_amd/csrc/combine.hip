@@ -397,14 +397,16 @@ static int shared_regime(const qmoe_config_t& c, int64_t N, int64_t rows, int64_
   // (qmm_dense_kernel addresses its activations with 32-bit byte offsets)
   return N * K <= kDenseMaxActs ? kRegimeDense : QMOE_REGIME_SMALL;
 }
-// Weights of one projection of all experts from which the hybrid regime runs its chains in phases.
-constexpr double kPhasedLayerWeights = 1e9;
 static int shared_gu_regime(const qmoe_config_t& c, int64_t N) {
   return shared_regime(c, N, 2 * static_cast<int64_t>(c.shared_inter), c.hidden, 6000000, 1e10);
 }
 static int shared_dn_regime(const qmoe_config_t& c, int64_t N) {
   return shared_regime(c, N, c.hidden, c.shared_inter, 4000000, 2.5e10);
 }
+
+// Weights of one projection of all experts from which the hybrid regime runs its chains in phases (measured
+// where the wait is).
+constexpr double kPhasedLayerWeights = 1e9;
 
 // Whether the router's logits above the decode sizes take the large kernel: beyond router_logits_kernel's one
 // 64-token tile per CU, but for a long K, which the large kernel's few tiles walk more slowly. Whole layers,
@@ -1160,8 +1162,12 @@ static int forward_impl(const qmoe_config_t* cfg, const qmoe_weights_t* wts, con
     rc = gate_up(kColdExperts);
     if (!rc) rc = gate_up(kHotExperts);
     // In large layers the cold down waits for the hot gate_up, beside which it would take compute units
-    // from the longer chain (c2 1000 tokens 890 -> 878 us per layer, 2000 tokens 1168 -> 1155); in small
-    // ones that costs more than it gives (c1 4096 skewed tokens 519 -> 536).
+    // from the longer chain. us per layer, without the wait and with it: c2 (2.1e9 weights a projection) int4 1000
+    // tokens 898 / 878, 2000 1143 / 1140, int6 1000 1293 / 1268, AWQ 2000 1349 / 1335; 256 experts 4096 x 1024 (1.07e9)
+    // int4 1000 551 / 547, int6 765 / 758; c3 (3.8e9) int6 2000 2893 / 2880, int4 1000 1651 / 1653. In smaller ones
+    // the wait costs more than it gives: 200 experts 3072 x 1536 (9.4e8) 1000 562 / 562, skewed 577 / 597; c1 (2.7e8)
+    // 600 185 / 196, 4096 451 / 458. (Skewed tokens lose by it in large layers too where the weights are int4, c2 2000
+    // 1166 / 1194, and gain with int6, 1597 / 1568; the host does not know the skew.)
     if (!rc && cstream != stream && static_cast<double>(c.n_experts) * c.inter * c.hidden >= kPhasedLayerWeights)
       rc = link(aux->hot, stream, aux->s, "hot gate_up");
     if (!rc) rc = down(kColdExperts);
