@@ -11,7 +11,8 @@
 //            shared weights' dtype                                     (:145-151)
 //   y = cast_x(routed + shared)                                        (:201-202)
 // as the reference's own float32 parity gates run it (parity/qwen35_forward_test.py:213-271:
-// hidden 32, group size 32, float32 throughout). Four launches (six with a shared expert): router, top-k,
+// hidden 32, group size 32, float32 throughout). Four launches (six with a shared expert, seven with a gated
+// one, whose logit is a product of its own): router, top-k,
 // gate_up with its gated activation, down with the combine; one wavefront per output (fixed-order
 // wavefront sums, fp32 accumulation), the affine weight s*q + b evaluated in fp32 per element from
 // the LSB-first packed code stream. These shapes are small (the parity configs); the fast path
@@ -46,34 +47,36 @@ struct GenW {
   int sb_dt, dense_dt, gshift, K;
 };
 
-// Every product is one wavefront per output (or per few outputs over the same activations): lane l
-// takes the 8-element pieces l, l + 64, ... of K, so that a row of 512 is one round of loads. At
-// these sizes the launch is a chain of dependent loads; element-strided lanes took eight rounds.
-// Elements 8c .. 8c + 7 of activation row `base` (element offset), rounded to act_round when that
-// differs from their dtype (the reference's cast to the weights' dtype); 0 past K.
-template <bool VEC>
-__device__ __forceinline__ void gen_x8(const void* act, int64_t base, int c, int K, int dt, int round,
-                                       float (&x)[8]) {
-  if (VEC) {   // (rows 16-byte aligned, K % 8 == 0)
-    if (dt == QMOE_DT_F32) {
-      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(static_cast<const float*>(act) + base + 8 * c);
-      const f32x4_t lo = p[0], hi = p[1];
+// Every product is one wavefront per output (or per few outputs over the same activations). At these sizes
+// the launch is a chain of dependent loads, so where K is a multiple of 8 (PIECES; packed K always is) lane l
+// takes the 8-element pieces l, l + 64, ... of K: a row of 512 is one round of loads, where element-strided
+// lanes took eight. Other K, dense only, keep the strided lanes: there a piece is eight scattered loads (100 x 60,
+// 200 bf16 tokens: 53 us per call, 108 in pieces).
+//
+// A piece is loaded as 16-byte words at its elements' alignment, since the caller's tensors may start anywhere:
+// global loads take any address (2048 x 1024 float32, 64 tokens, tensors 4 bytes off: 852 us, 4478 element by
+// element).
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
+
+// Elements 8c .. 8c + 7 of the row at element offset `base`, rounded to `round` when that differs from
+// their dtype (the reference's cast to the weights' dtype).
+__device__ __forceinline__ void gen_x8(const void* act, int64_t base, int c, int dt, int round, float (&x)[8]) {
+  if (dt == QMOE_DT_F32) {
+    const f32x4_u* p = reinterpret_cast<const f32x4_u*>(static_cast<const float*>(act) + base + 8 * c);
+    const f32x4_u lo = p[0], hi = p[1];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        x[j] = lo[j];
-        x[4 + j] = hi[j];
-      }
-    } else {
-      const u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(act) + base + 8 * c);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        x[2 * j] = bf16lo_to_f32(v[j]);
-        x[2 * j + 1] = bf16hi_to_f32(v[j]);
-      }
+    for (int j = 0; j < 4; ++j) {
+      x[j] = lo[j];
+      x[4 + j] = hi[j];
     }
   } else {
+    const u32x4_u v = *reinterpret_cast<const u32x4_u*>(static_cast<const uint16_t*>(act) + base + 8 * c);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = (8 * c + j < K) ? gen_ld(act, base + 8 * c + j, dt) : 0.f;
+    for (int j = 0; j < 4; ++j) {
+      x[2 * j] = bf16lo_to_f32(v[j]);
+      x[2 * j + 1] = bf16hi_to_f32(v[j]);
+    }
   }
   if (round != dt) {
 #pragma unroll
@@ -83,7 +86,7 @@ __device__ __forceinline__ void gen_x8(const void* act, int64_t base, int c, int
 
 // acc + x . W[row][8c .. 8c + 7], the affine weight fma(s, q, b) formed in fp32 per element. Eight
 // codes of any width start on a byte and span at most two words.
-template <int BITS, bool VEC>
+template <int BITS>
 __device__ __forceinline__ float gen_dot8(const GenW& w, int64_t row, int c, const float (&x)[8], float acc) {
   if constexpr (BITS > 0) {
     const uint32_t* p = w.packed + row * (static_cast<int64_t>(w.K) * BITS / 32);
@@ -100,11 +103,34 @@ __device__ __forceinline__ float gen_dot8(const GenW& w, int64_t row, int c, con
     }
   } else {
     float y[8];
-    gen_x8<VEC>(w.dense, row * w.K, c, w.K, w.dense_dt, w.dense_dt, y);
+    gen_x8(w.dense, row * w.K, c, w.dense_dt, w.dense_dt, y);
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc = fmaf(x[j], y[j], acc);
   }
   return acc;
+}
+
+// This lane's part of x . W_i[rows[i]] (i < M): x the row at element offset `base`, rounded to `round`.
+template <int BITS, bool PIECES, int M>
+__device__ __forceinline__ void gen_dots(const void* act, int64_t base, int dt, int round, const GenW* const (&w)[M],
+                                         const int64_t (&rows)[M], int lane, float (&acc)[M]) {
+  static_assert(PIECES || BITS == 0, "packed rows are whole pieces");
+  const int K = w[0]->K;
+  if constexpr (PIECES) {
+    for (int c = lane; 8 * c < K; c += 64) {
+      float x[8];
+      gen_x8(act, base, c, dt, round, x);
+#pragma unroll
+      for (int i = 0; i < M; ++i) acc[i] = gen_dot8<BITS>(*w[i], rows[i], c, x, acc[i]);
+    }
+  } else {
+    for (int k = lane; k < K; k += 64) {
+      float x = gen_ld(act, base + k, dt);
+      if (round != dt) x = gen_round(x, round);
+#pragma unroll
+      for (int i = 0; i < M; ++i) acc[i] = fmaf(x, gen_ld(w[i]->dense, rows[i] * K + k, w[i]->dense_dt), acc[i]);
+    }
+  }
 }
 
 template <int M>
@@ -129,7 +155,7 @@ struct GenMv {
   int col0;
 };
 
-template <bool VEC>
+template <bool PIECES>
 __global__ void __launch_bounds__(256) gen_matvec_kernel(GenMv a) {
   const int lane = threadIdx.x & 63;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
@@ -137,11 +163,7 @@ __global__ void __launch_bounds__(256) gen_matvec_kernel(GenMv a) {
   const int64_t r = gid / a.n_out;
   const int o = static_cast<int>(gid - r * a.n_out);
   float acc[1] = {0.f};
-  for (int c = lane; 8 * c < a.w.K; c += 64) {
-    float x[8];
-    gen_x8<VEC>(a.act, r * a.w.K, c, a.w.K, a.act_dt, a.act_round, x);
-    acc[0] = gen_dot8<0, VEC>(a.w, o, c, x, acc[0]);
-  }
+  gen_dots<0, PIECES, 1>(a.act, r * a.w.K, a.act_dt, a.act_round, {&a.w}, {o}, lane, acc);
   gen_wave_sum(acc);
   if (lane == 0) gen_st(a.out, r * a.ld_out + a.col0 + o, acc[0], a.out_dt);
 }
@@ -162,7 +184,7 @@ struct GenGu {
   float alpha, limit;
 };
 
-template <int BITS, bool VEC>
+template <int BITS, bool PIECES>
 __global__ void __launch_bounds__(256) gen_gate_up_kernel(GenGu a) {
   const int lane = threadIdx.x & 63;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
@@ -173,12 +195,8 @@ __global__ void __launch_bounds__(256) gen_gate_up_kernel(GenGu a) {
   const int64_t row = static_cast<int64_t>(e) * a.n2 + i;
   const int64_t base = r / a.row_div * a.w.K;
   float v[2] = {0.f, 0.f};
-  for (int c = lane; e >= 0 && 8 * c < a.w.K; c += 64) {
-    float x[8];
-    gen_x8<VEC>(a.act, base, c, a.w.K, a.act_dt, a.act_round, x);
-    v[0] = gen_dot8<BITS, VEC>(a.w, row, c, x, v[0]);
-    v[1] = gen_dot8<BITS, VEC>(a.w_up, row + a.up, c, x, v[1]);
-  }
+  if (e >= 0)
+    gen_dots<BITS, PIECES, 2>(a.act, base, a.act_dt, a.act_round, {&a.w, &a.w_up}, {row, row + a.up}, lane, v);
   gen_wave_sum(v);
   if (lane == 0)
     gen_st(a.h, r * a.n + i, glu_f(gen_round(v[0], a.dt), gen_round(v[1], a.dt), a.glu, a.alpha, a.limit), a.dt);
@@ -201,7 +219,7 @@ struct GenDn {
   int y_dt;
 };
 
-template <int BITS, bool VEC>
+template <int BITS, bool PIECES>
 __global__ void __launch_bounds__(256) gen_down_combine_kernel(GenDn a) {
   const int lane = threadIdx.x & 63;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
@@ -214,17 +232,14 @@ __global__ void __launch_bounds__(256) gen_down_combine_kernel(GenDn a) {
     float v[SB];
 #pragma unroll
     for (int i = 0; i < SB; ++i) {
-      v[i] = 0.f;
+      float d[1] = {0.f};
       if (s0 + i < a.k) {
         const int64_t m = t * a.k + s0 + i;
         const int e = a.idx[m];
-        const int64_t row = static_cast<int64_t>(e) * a.H + j;
-        for (int c = lane; e >= 0 && 8 * c < a.w.K; c += 64) {
-          float x[8];
-          gen_x8<VEC>(a.h, m * a.w.K, c, a.w.K, a.dt, a.dt, x);
-          v[i] = gen_dot8<BITS, VEC>(a.w, row, c, x, v[i]);
-        }
+        if (e >= 0)
+          gen_dots<BITS, PIECES, 1>(a.h, m * a.w.K, a.dt, a.dt, {&a.w}, {static_cast<int64_t>(e) * a.H + j}, lane, d);
       }
+      v[i] = d[0];
     }
     gen_wave_sum(v);
 #pragma unroll
@@ -237,13 +252,6 @@ __global__ void __launch_bounds__(256) gen_down_combine_kernel(GenDn a) {
   }
 }
 
-// 16-byte loads of activation and dense weight rows need whole 8-element pieces and aligned bases;
-// anything else (the caller's tensors may start anywhere) loads element by element.
-static bool gen_vec(int K, const void* a, const void* b = nullptr, const void* c = nullptr) {
-  const uintptr_t bits = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c);
-  return K % 8 == 0 && bits % 16 == 0;
-}
-
 static int gen_grid(int64_t waves, unsigned* grid) {
   if ((waves + 3) / 4 > 0x7fffffff) return fail("general: product too large");
   *grid = static_cast<unsigned>((waves + 3) / 4);
@@ -254,22 +262,25 @@ static int gen_matvec(const GenMv& a, hipStream_t stream) {
   unsigned grid;
   if (int rc = gen_grid(a.rows * a.n_out, &grid)) return rc;
   if (!grid) return 0;
-  if (gen_vec(a.w.K, a.act, a.w.dense)) gen_matvec_kernel<true><<<grid, 256, 0, stream>>>(a);
+  if (a.w.K % 8 == 0) gen_matvec_kernel<true><<<grid, 256, 0, stream>>>(a);
   else gen_matvec_kernel<false><<<grid, 256, 0, stream>>>(a);
   return check_launch("general matvec");
 }
 
-// launch KERNEL<bits, vec> for a code width (0: dense)
-#define QMOE_GEN(KERNEL, bits, vec, grid, stream, a)                                                          \
+// launch KERNEL<bits, pieces> for a code width (0: dense)
+#define QMOE_GEN(KERNEL, bits, grid, stream, a)                                                               \
   do {                                                                                                        \
     switch (bits) {                                                                                           \
-      case 0: if (vec) KERNEL<0, true><<<grid, 256, 0, stream>>>(a); else KERNEL<0, false><<<grid, 256, 0, stream>>>(a); break; \
-      case 2: if (vec) KERNEL<2, true><<<grid, 256, 0, stream>>>(a); else KERNEL<2, false><<<grid, 256, 0, stream>>>(a); break; \
-      case 3: if (vec) KERNEL<3, true><<<grid, 256, 0, stream>>>(a); else KERNEL<3, false><<<grid, 256, 0, stream>>>(a); break; \
-      case 4: if (vec) KERNEL<4, true><<<grid, 256, 0, stream>>>(a); else KERNEL<4, false><<<grid, 256, 0, stream>>>(a); break; \
-      case 5: if (vec) KERNEL<5, true><<<grid, 256, 0, stream>>>(a); else KERNEL<5, false><<<grid, 256, 0, stream>>>(a); break; \
-      case 6: if (vec) KERNEL<6, true><<<grid, 256, 0, stream>>>(a); else KERNEL<6, false><<<grid, 256, 0, stream>>>(a); break; \
-      case 8: if (vec) KERNEL<8, true><<<grid, 256, 0, stream>>>(a); else KERNEL<8, false><<<grid, 256, 0, stream>>>(a); break; \
+      case 0:                                                                                                 \
+        if (a.w.K % 8 == 0) KERNEL<0, true><<<grid, 256, 0, stream>>>(a);                                     \
+        else KERNEL<0, false><<<grid, 256, 0, stream>>>(a);                                                   \
+        break;                                                                                                \
+      case 2: KERNEL<2, true><<<grid, 256, 0, stream>>>(a); break;                                            \
+      case 3: KERNEL<3, true><<<grid, 256, 0, stream>>>(a); break;                                            \
+      case 4: KERNEL<4, true><<<grid, 256, 0, stream>>>(a); break;                                            \
+      case 5: KERNEL<5, true><<<grid, 256, 0, stream>>>(a); break;                                            \
+      case 6: KERNEL<6, true><<<grid, 256, 0, stream>>>(a); break;                                            \
+      case 8: KERNEL<8, true><<<grid, 256, 0, stream>>>(a); break;                                            \
       default: return fail("general: bits must be 2, 3, 4, 5, 6 or 8");                                       \
     }                                                                                                         \
   } while (0)
@@ -278,16 +289,14 @@ static int gen_gate_up(const GenGu& a, int bits, hipStream_t stream) {
   unsigned grid;
   if (int rc = gen_grid(a.rows * a.n, &grid)) return rc;
   if (!grid) return 0;
-  const bool vec = gen_vec(a.w.K, a.act, bits ? nullptr : a.w.dense, bits ? nullptr : a.w_up.dense);
-  QMOE_GEN(gen_gate_up_kernel, bits, vec, grid, stream, a);
+  QMOE_GEN(gen_gate_up_kernel, bits, grid, stream, a);
   return check_launch("general gate_up");
 }
 
 static int gen_down_combine(const GenDn& a, int bits, hipStream_t stream) {
   unsigned grid;
   if (int rc = gen_grid(a.N * a.H, &grid)) return rc;
-  const bool vec = gen_vec(a.w.K, a.h, bits ? nullptr : a.w.dense);
-  QMOE_GEN(gen_down_combine_kernel, bits, vec, grid, stream, a);
+  QMOE_GEN(gen_down_combine_kernel, bits, grid, stream, a);
   return check_launch("general down + combine");
 }
 

@@ -1,11 +1,11 @@
 """GPU tier: the 16-byte-piece kernels of the reference-dtype block (general.hip) and of the fp32 router
-(router.hip), at the sizes where their pieces end: rows that are not whole pieces or not whole
-wavefront rounds, one piece, more than one round, every code width across word boundaries, and bases
-off 16 bytes, which take the element-wise form.
+(router.hip), at the sizes where their pieces end: rows that are not whole pieces (element-strided
+lanes) or not whole wavefront rounds, one piece, more than one round, every code width across word
+boundaries, and bases off 16 bytes (the router's take its element-wise form).
 
 Bars: float32 results within 1e-5 of float64 (scaled by max(1, max|y|); K <= 1096 fp32 sums of
 O(1) terms stay below 2e-6), as tests/test_gpu_12_general.py; an unaligned copy of the same data
-gives the same bits (same pieces, same order of sums).
+gives the same bits (same order of sums).
 """
 
 from __future__ import annotations
