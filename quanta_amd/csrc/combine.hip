@@ -375,7 +375,7 @@ static bool large_ok(const qmoe_config_t& c, int64_t N) { return N > 256 && c.hi
 // that do not depend on the batch), above that qmm_dense_kernel's 64 x 64 tiles, which fill the chip with
 // small products, and the large kernel's 128 x 256 tiles where about 100 of them (3e6 outputs) do as well and
 // their fewer bytes from L2 win. The gate_up runs beside the routing chain, which the large tiles hold up, so
-// it also takes 1e10 multiply-adds, or twice the outputs; the down runs beside the hot experts and is half
+// it also takes 1.35e10 multiply-adds, or twice the outputs; the down runs beside the hot experts and is half
 // the work. Fewer than 640 tokens leave too much of the 128-token tiles empty. Whole layers, us, int8 weights
 // (bf16 alike), 64 x 64 against 128 x 256 tiles (hidden x shared intermediate at tokens):
 //   gate_up  7168 x 2048 600 1453 / 1502, 800 1531 / 1559, 1000 1695 / 1685, 1500 2079 / 2001; 4096 x 1024 1000
@@ -398,7 +398,7 @@ static int shared_regime(const qmoe_config_t& c, int64_t N, int64_t rows, int64_
   return N * K <= kDenseMaxActs ? kRegimeDense : QMOE_REGIME_SMALL;
 }
 static int shared_gu_regime(const qmoe_config_t& c, int64_t N) {
-  return shared_regime(c, N, 2 * static_cast<int64_t>(c.shared_inter), c.hidden, 6000000, 1e10);
+  return shared_regime(c, N, 2 * static_cast<int64_t>(c.shared_inter), c.hidden, 6000000, 1.35e10);
 }
 static int shared_dn_regime(const qmoe_config_t& c, int64_t N) {
   return shared_regime(c, N, c.hidden, c.shared_inter, 4000000, 2.5e10);
@@ -408,12 +408,13 @@ static int shared_dn_regime(const qmoe_config_t& c, int64_t N) {
 // where the wait is).
 constexpr double kPhasedLayerWeights = 1e9;
 
-// Whether the router's logits above the decode sizes take the large kernel: beyond router_logits_kernel's one
-// 64-token tile per CU, but for a long K, which the large kernel's few tiles walk more slowly. Whole layers,
-// us, router_logits_kernel against the large kernel: c1 2048 tokens 279 / 291, 4096 457 / 443, 8192 750 / 722;
-// c2 1536 981 / 994, 2000 1114 / 1114, 3000 1333 / 1319, 4096 1594 / 1578; c3 2500 2541 / 2592, 4096 3805 / 3881.
+// Whether the router's logits above the decode sizes take the large kernel: well beyond router_logits_kernel's
+// one 64-token tile per CU, but for a long K, which the large kernel's few tiles walk more slowly. Whole
+// layers, us, router_logits_kernel against the large kernel: c1 2048 tokens 271 / 290, 4096 416 / 441, 6000 600 / 585,
+// 8192 734 / 712; c2 1000 865 / 887, 2000 1103 / 1104, 3000 1326 / 1316, 6000 2156 / 2137; 512 experts of hidden 2048
+// 3000 454 / 462, 6000 736 / 743; c3 2500 2502 / 2553, 6000 5082 / 5162; 128 of hidden 3072 8192 2232 / 2274.
 static bool router_large(const qmoe_config_t& c, int64_t N, int64_t rows) {
-  return large_ok(c, N) && c.hidden <= 4096 && (N + 63) / 64 * ((rows + 63) / 64) > 256;
+  return large_ok(c, N) && c.hidden <= 4096 && (N + 63) / 64 * ((rows + 63) / 64) > 400;
 }
 
 // Whether a projection of an int8 shared expert is expanded to bf16 for this call: the large-M

@@ -622,22 +622,26 @@ __global__ void __launch_bounds__(kPfThreads) qmm_large_kernel(QmmArgs a) {
 // ============================================================================ router logits
 // Logits of batches above the decode sizes, short of those that fill the chip with qmm_large_kernel's tiles:
 // 16 MB tokens x 64 weight rows per workgroup, a 128-deep k superblock per iteration, two 16x16 blocks per
-// wavefront (weight tile w % 4, m-blocks 2 (w / 4) and the next), tokens and weights through an LDS ring
-// ([16-row block][step][64 lanes] x 16 B).
+// wavefront (weight tile w % 4, m-blocks 2 (w / 4) and the next), tokens and weights through an LDS ring of
+// [16-row block][step] x 1 KiB: a weight tile's fragments as they are stored; of a token block 64 bytes of each
+// row, loaded by four neighbouring lanes, 16-byte chunk c at c ^ (row / 4 % 4), which spreads the fragment
+// reads over all banks.
 //
 // Every logit is one accumulator over all of K in k order, which is qmm_large_kernel's sum: the expert ids of a
 // prompt depend on neither the kernel that a batch size takes nor K's split over wavefronts, whose sums
 // differ by up to 8e-6 at c2 and move a token across a tie of its last expert now and then.
 //
-// What bounds it is the latency of the loads, K / 128 dependent rounds: the ring keeps them NS - 1 superblocks
-// ahead.
+// What bounds it is latency, K / 128 rounds of a barrier, fragment reads and dependent MFMAs with the loads NS - 1
+// superblocks ahead. us, the large kernel before, now: 2048 x 256 391 tokens 25 / 9.1, 2048 29 / 9.8; 4096 x 512 300
+// 45 / 15, 1000 46 / 16, 2000 48 / 21; 7168 x 256 800 76 / 24, 2300 108 / 43. (32-token tiles with six slots: the same,
+// and 144 KiB that no other workgroup can share. Lanes that load 16 bytes of 16 rows each: 2300 49.)
 template <int MB>
 struct RouterCfg {
   static constexpr int WAVES = 2 * MB;                       // MB = 2 or 4
   static constexpr int SLOT = (MB + 4) * 4096;               // one superblock: MB token blocks, 4 weight tiles
-  static constexpr int NS = (MB == 2) ? 6 : 4;
+  static constexpr int NS = (MB == 2) ? 3 : 4;
   static constexpr int LOADS = 2 + 16 / WAVES;               // per wavefront and superblock
-  static constexpr size_t LDS = static_cast<size_t>(NS) * SLOT;   // 144 or 128 KiB
+  static constexpr size_t LDS = static_cast<size_t>(NS) * SLOT;   // 72 or 128 KiB
 };
 
 template <int MB>
@@ -657,8 +661,9 @@ __global__ void __launch_bounds__(64 * RouterCfg<MB>::WAVES) router_logits_kerne
   // (never stored).
   const int ab = (MB == 2) ? wave >> 1 : wave & 3, as = 2 * ((MB == 2) ? wave & 1 : wave >> 2);
   const int ws = (16 / C::WAVES) * (wave >> 2);
-  const int t = 16 * MB * tb + 16 * ab + (lane & 15);
-  const char* xp = reinterpret_cast<const char*>(a.act + (t < rows ? t : 0) * static_cast<int64_t>(a.K)) + 16 * (lane >> 4);
+  const int t = 16 * MB * tb + 16 * ab + (lane >> 2);
+  const char* xp = reinterpret_cast<const char*>(a.act + (t < rows ? t : 0) * static_cast<int64_t>(a.K)) +
+                   16 * ((lane & 3) ^ ((lane >> 4) & 3));
   const char* wp = static_cast<const char*>(a.codes) + (4 * rb + (wave & 3)) * static_cast<int64_t>(a.K / 32) * 1024;
   const uint32_t lds_base = lds_offset(lds);
   auto issue = [&](int p) __attribute__((always_inline)) {
@@ -672,6 +677,7 @@ __global__ void __launch_bounds__(64 * RouterCfg<MB>::WAVES) router_logits_kerne
   const int n0 = min(C::NS - 1, nsb);
   for (int p = 0; p < n0; ++p) issue(p);
   const int mb = 2 * (wave >> 2);
+  const int xo = 4 * (lane & 15) + ((lane >> 4) ^ ((lane >> 2) & 3));   // the lane's fragment in a token block's step
   f32x4_t acc[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -681,12 +687,12 @@ __global__ void __launch_bounds__(64 * RouterCfg<MB>::WAVES) router_logits_kerne
     if (p + C::NS - 2 < nsb) wait_vmcnt<(C::NS - 2) * C::LOADS>(); else wait_vmcnt<0>();
     lg_barrier();
     if (p + C::NS - 1 < nsb) issue(p + C::NS - 1);
-    const u32x4* sl = reinterpret_cast<const u32x4*>(lds_c + p % C::NS * C::SLOT) + lane;
+    const u32x4* sl = reinterpret_cast<const u32x4*>(lds_c + p % C::NS * C::SLOT);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const bf16x8_t B = as_bf16x8(sl[256 * (MB + (wave & 3)) + 64 * s]);
+      const bf16x8_t B = as_bf16x8(sl[256 * (MB + (wave & 3)) + 64 * s + lane]);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) acc[i] = mfma16(as_bf16x8(sl[256 * (mb + i) + 64 * s]), B, acc[i]);
+      for (int i = 0; i < 2; ++i) acc[i] = mfma16(as_bf16x8(sl[256 * (mb + i) + 64 * s + xo]), B, acc[i]);
     }
   }
 #pragma unroll
@@ -716,9 +722,9 @@ int launch_router_logits(const QmmArgs& a, hipStream_t stream) {
     return fail("router logits: one dense bf16 segment");
   if (a.K <= 0 || a.K % 128 || a.n_rows <= 0 || a.n_rows % 64)
     return fail("router logits: K % 128 == 0 and weight rows % 64 == 0 required");
-  // 32-token tiles while they are at most a workgroup per CU (us, 32 against 64 tokens: c2 1000 tokens 16 / 22,
-  // c1 391 10 / 12, c1 2048 11 / 13, 7168 x 256 700 17 / 21), 64-token ones above, where a second wave of the
-  // smaller ones would read a third more (c2 1536 30 / 23).
+  // 32-token tiles while they are at most one workgroup per CU, 64-token ones above, where the smaller ones would
+  // read a third more. us, 32 against 64 tokens: 2048 x 256 391 9.1 / 12, 2048 9.8 / 12, 3000 12.9 / 11.6; 4096 x 512 1000
+  // 16.5 / 18, 1500 23 / 20; 7168 x 256 800 24 / 28, 1500 27 / 31, 2300 45 / 43.
   const bool two = (a.dense_rows + 31) / 32 * (a.n_rows / 64) <= 256;
   return two ? launch_router_k<2>(a, stream) : launch_router_k<4>(a, stream);
 }
