@@ -7,8 +7,9 @@ The reference's loader dequantizes it to bf16 at load (src/quanta/qwen35/artifac
 so the bars are:
   - bit-identical to the same block with the shared expert given as its bf16 dequant, at every
     batch size and through every path (pair launch with and without the fused RMSNorm, the
-    fused combine + shared down, the unfused small-regime launches above 64 tokens, the expanded
-    bf16 copy of the large regime above 256 tokens, the allocation-free entry point);
+    fused combine + shared down, the unfused small-regime launches above 64 tokens, the dense kernel
+    above 256 tokens, the expanded bf16 copies of the projections that the large kernel takes, the
+    allocation-free entry point);
   - the block against the oracle (oracle.moe.shared_weight dequantizes the triplets) within the
     BASELINE gates, with the shared expert carrying most of the output.
 """
@@ -73,7 +74,7 @@ def test_tiled_int8_products_match_bf16(gpu):
 def test_block_int8_shared_equals_bf16_dequant(gpu, N):
     """c1-shaped block (H 2048, Is 512): the int8 shared expert gives the bf16-dequant block's
     outputs bit for bit through the decode launches (N <= 64 fused, 65-256 unfused small regime)
-    and the large regime's expanded copy (N > 256)."""
+    and the dense kernel (N > 256; the expanded copies: test_expanded_projections)."""
     s = _spec("c1")
     p8, p16 = _pair(s, gpu, seed=21)
     x = synth.make_inputs(s, N, device=gpu, seed=N)[None]
@@ -136,3 +137,26 @@ def test_int8_shared_vs_oracle(gpu, N):
     print(f"[parity] int8 shared N={N}: shared part {share:.2f} of |y|", flush=True)
     assert share > 0.5
     assert_close(f64(y), it["y_exact"], f"int8 shared N={N}")
+
+
+@pytest.mark.parametrize("N,H,Is", [(639, 6400, 2432), (640, 6400, 2432), (641, 6400, 128), (700, 1024, 4736)])
+def test_expanded_projections(gpu, N, H, Is):
+    """Either side of the large kernel's line, for each projection by itself: neither on it (dense kernel, codes
+    read in registers), both, the down only, the gate_up only (expanded to bf16 in the workspace). Equal to
+    the bf16-dequant block bit for bit, and to the oracle within the gates with the shared expert carrying
+    most of the output."""
+    s = _spec("c1", hidden_size=H, num_experts=8, num_experts_per_tok=2, moe_intermediate_size=128,
+              shared_expert_intermediate_size=Is)
+    p8 = synth.make_layer(s, device=gpu, seed=N)
+    for key in SHARED:
+        # (outputs of order 1: gate and up of deviation 1, the down's sums over Is of deviation 0.6)
+        w = p8[key].float() * (50.0 / p8[key].shape[1] ** 0.5)
+        pk, sc, bi = quantize_affine(w.to(torch.bfloat16), 8, group_size=64)
+        p8[key] = {"packed": pk, "scale": sc, "bias": bi, "group_size": 64, "bits": 8}
+    x = synth.make_inputs(s, N, device=gpu, seed=11 + N)
+    y8 = qwen35_moe(x[None], p8, s.cfg)[0]
+    y16 = qwen35_moe(x[None], _dequant_shared(p8), s.cfg)[0]
+    assert torch.equal(y8, y16), f"max diff {(y8.float() - y16.float()).abs().max().item()}"
+    _, it = om.moe_forward(f64(x), oracle_params_from_torch(p8), k=2, inter=128)
+    assert float(abs(it["shared"]).mean() / abs(it["y_exact"]).mean()) > 0.5
+    assert_close(f64(y8), it["y_exact"], f"expanded N={N} H={H} Is={Is}")

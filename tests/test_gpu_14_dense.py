@@ -71,9 +71,9 @@ def test_router_logits_keep_their_order(gpu, N, H, E):
 
 @pytest.mark.parametrize("E,N", [(64, 300), (32, 400), (8, 300)])
 def test_two_chains_repeat_bit_for_bit(gpu, E, N):
-    """The hot and cold experts' chains run on two streams over disjoint rows: repeated calls on
-    one workspace, on two streams, give the same bits (mean rows per expert 9, 25 and 75: the cold
-    chain, then the hot one on the caller's stream)."""
+    """The hot and cold experts' chains run on two streams over disjoint rows: calls on one stream after
+    another, each waited for, give the same bits (mean rows per expert 9, 25 and 75: the cold chain, then the hot
+    one on the caller's stream)."""
     s = synth.scaled_spec("c1", hidden_size=512, num_experts=E, num_experts_per_tok=2,
                           moe_intermediate_size=256, shared_expert_intermediate_size=256)
     p = synth.make_layer(s, device=gpu, seed=E)
@@ -90,3 +90,28 @@ def test_two_chains_repeat_bit_for_bit(gpu, E, N):
             y = qwen35_moe(x, p, s.cfg)
             torch.cuda.synchronize()
         assert torch.equal(y, want), i
+
+
+@pytest.mark.parametrize("H,I,E,k,N", [(512, 256, 64, 2, 300), (512, 256, 8, 2, 300), (2048, 512, 256, 8, 391),
+                                       (2048, 512, 256, 8, 600), (4096, 1024, 256, 4, 600)])
+def test_two_chains_of_concurrent_callers(gpu, H, I, E, k, N):
+    """Two callers' streams, other inputs on each and no wait between their calls, share the auxiliary stream and
+    its events: every output is the serial call's, bit for bit, and that is the decode kernels' within the gates
+    (hot chain on the auxiliary stream, on the caller's, and, from 1e9 weights, in phases)."""
+    s = synth.scaled_spec("c1", hidden_size=H, num_experts=E, num_experts_per_tok=k,
+                          moe_intermediate_size=I, shared_expert_intermediate_size=256)
+    p = synth.make_layer(s, device=gpu, seed=E)
+    xs = [synth.make_inputs(s, N, device=gpu, seed=N + i)[None] for i in range(2)]
+    want = [qwen35_moe(x, p, s.cfg) for x in xs]
+    small = [qwen35_moe(x, p, s.cfg, regime=L.REGIME_SMALL) for x in xs]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    outs = []
+    for i in range(8):
+        with torch.cuda.stream(streams[i % 2]):
+            outs.append(qwen35_moe(xs[i % 2], p, s.cfg))
+    torch.cuda.synchronize()
+    for i, y in enumerate(outs):
+        assert torch.equal(y, want[i % 2]), f"call {i}"
+    for w, r in zip(want, small):
+        assert_close(f64(w[0]), f64(r[0]), f"two chains H={H} E={E} N={N} vs decode kernels", want_rounded=True)

@@ -62,6 +62,23 @@ def test_dense_float32_pieces(gpu, H, I):
     assert torch.equal(qwen35_moe(_off(d(x)[None]), q, cfg)[0], y)
 
 
+@pytest.mark.parametrize("H,I", [(40, 24), (1000, 504), (100, 60)])
+def test_dense_bf16_off_alignment(gpu, H, I):
+    """bf16 tensors two bytes off give the aligned ones' bits (whole pieces; element-strided lanes)."""
+    g = torch.Generator(device="cpu").manual_seed(H)
+    r = lambda *s: (torch.randn(*s, generator=g) / s[-1] ** 0.5).to(torch.bfloat16).to(gpu)
+    p = {"gate": r(E, H), "experts_gate_up": r(E, 2 * I, H), "experts_down": r(E, H, I)}
+    x = r(1, 5, H) * H ** 0.5
+    cfg = MoEConfig(H, E, K_TOP, I, 0)
+    y = qwen35_moe(x, p, cfg)
+    d = lambda t: t.double().cpu().numpy()
+    want = _ref(d(x)[0], *(d(p[k]) for k in ("gate", "experts_gate_up", "experts_down")), I)
+    # gate, up, h and the down rows each round to bf16 (2^-9 relative), the output once more
+    assert np.linalg.norm(d(y)[0] - want) <= 1e-2 * np.linalg.norm(want)
+    q = {key: _off(v) for key, v in p.items()}
+    assert torch.equal(qwen35_moe(_off(x), q, cfg), y)
+
+
 @pytest.mark.parametrize("bits,gs,H,I", [(2, 32, 32, 32), (3, 32, 96, 544), (4, 64, 576, 64), (5, 32, 544, 32),
                                          (6, 128, 640, 128), (8, 32, 32, 64)])
 def test_packed_float32_pieces(gpu, bits, gs, H, I):
