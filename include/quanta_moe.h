@@ -75,9 +75,9 @@ extern "C" {
 /* grouped-qmm regimes */
 #define QMOE_REGIME_AUTO 0
 #define QMOE_REGIME_SMALL 1 /* 16-token m-tiles, weights streamed to registers (decode) */
-#define QMOE_REGIME_LARGE 2 /* prefill: experts of > 16 rows on 128-row LDS-staged fp16 tiles
-                               (128x512 for int4 weights in 512-row blocks, else 128x256),
-                               the others on 16-token m-tiles */
+#define QMOE_REGIME_LARGE 2 /* prefill: experts of more than 16 rows (32 while few experts have as
+                               many) on 128-row LDS-staged fp16 tiles (128x512 for int3/int4 weights
+                               in 512-row blocks, else 128x256), the others on 16-token m-tiles */
 
 /* gated activation of the SwiGLU epilogue, h = act(gate, up) on the bf16 gate/up values in fp32:
  *  SILU        silu(g) * u                                (src/quanta/qwen35/moe.py:59-63)
@@ -134,8 +134,9 @@ typedef struct {
                             int8 weights are dequantized in registers to bf16(s*q + b), the bf16
                             weights the reference's loader makes of them
                             (src/quanta/qwen35/artifact.py:105-115), so both formats give the same
-                            outputs; int8 reads half the bytes. Above 256 tokens the block first
-                            expands them into its workspace. */
+                            outputs; int8 reads half the bytes. In prompts of 640 tokens or more
+                            the block first expands a projection into its workspace where that
+                            projection's product is large enough for the 128x256 bf16 tiles. */
 } qmoe_config_t;
 
 /* Prepared (resident) weights of one block; every array is device memory. */

@@ -166,8 +166,9 @@ __device__ __forceinline__ uint32_t deq_pair3(uint32_t w0, uint32_t w1, uint32_t
 // PFLOP/s, what a large library product reaches on this card.
 //
 // All streaming loads go global -> LDS directly (global_load_lds_dwordx4 / _dword, inline assembly), into
-// a ring of two slots of one superblock each, three for tiles of up to 64 rows, whose activations leave
-// the room: loads one or two superblocks ahead, issued between the MFMAs. At the end of superblock p every
+// a ring of slots of one superblock each, three wherever they fit in LDS (PfCfg::slots: tiles of any size for
+// int3 and int4 with NB = 1, up to 96 rows for int6 and for int3 with NB = 2, up to 64 for int4 with NB = 2), else
+// two: loads one or two superblocks ahead, issued between the MFMAs. At the end of superblock p every
 // wavefront waits for its own loads of p+1, and one barrier publishes slot p+1 and retires slot p. A
 // slot holds
 //  * A, 8 KiB per m-block: wavefront w loads rows 16w .. 16w+15, a 64-byte piece q (16-byte chunks 4q .. 4q+3

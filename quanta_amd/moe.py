@@ -574,8 +574,8 @@ def _prepare_mixed(p: dict, cfg, *, topk, regime) -> Prepared:
 
 
 def _dense_regime(n: int, hidden: int) -> int:
-    """Regime of the op-level dense (router / shared expert) matmuls (qmoe_forward has a third
-    kernel for them above 256 tokens, dense.hip)."""
+    """Regime of the op-level dense (router / shared expert) matmuls (qmoe_forward has
+    kernels of its own for them above 256 tokens: prefill.hip's router logits, dense.hip)."""
     return L.REGIME_LARGE if (n > 256 and hidden % 256 == 0) else L.REGIME_SMALL
 
 

@@ -328,8 +328,8 @@ def test_prefill_zipf_c4(gpu):
 
 def test_prefill_chunking_contract_c4(gpu):
     """Above 256 tokens (the hybrid large-M regime) a token's output depends on which kernel ran
-    each of its experts: experts routed more than 16 rows of the call run on the MFMA prefill
-    kernels (fp16-dequantized weights), the others on the decode kernel (bf16 codes, the affine
+    each of its experts: experts routed more than 16 rows of the call (32 where few are, as in the
+    calls of 300 tokens here) run on the MFMA prefill kernels (fp16-dequantized weights), the others on the decode kernel (bf16 codes, the affine
     map on the products). Chunking the call changes those row counts, so the reference's batch
     invariance (src/quanta/qwen35/moe.py:97-100; its chunk gate, parity/moe_chunk_test.py:47-62)
     holds here within the parity gates, not bit for bit. The whole 4096-token Zipf call and the

@@ -321,9 +321,9 @@ def test_block_int3_large_regime_vs_oracle(gpu, gs, gu_bits, dn_bits, E, N, I):
     """int3 layers above 256 tokens (Kimi's gate/up int3 + down int4 at group 128, and int3
     throughout): hot experts on the prefill kernels, the rest on the decode kernel (E = 32 at 300
     tokens holds both); against the oracle and against the decode kernel's output. I = 256 runs
-    the int3 stacks on the 256-row kernel; I = 512 gives gate_up 1024 rows, a multiple of 512, so
-    the 512-row int3 kernel (qmm_wide_int3_kernel) takes it, and with int3 down (H = 512 rows)
-    the down projection too, both over the hybrid regime's tile maps."""
+    the int3 stacks on the 256-row tile (prefill_kernel, NB = 1); I = 512 gives gate_up 1024 rows, a
+    multiple of 512, so the 512-row tile (NB = 2) takes it, and with int3 down (H = 512 rows) the
+    down projection too, both over the hybrid regime's tile maps."""
     cfg = MoEConfig(512, E, 2, I, 256)
     p = _layer_widths(gpu, gs, 13 * N + gs + I, gu_bits, dn_bits, E=E, I=I)
     x = _inputs(gpu, N, 512, N)

@@ -45,7 +45,7 @@ def test_noalloc_decode_c2(gpu):
 
 
 def test_noalloc_hybrid_prefill(gpu):
-    """A small layer at 600 tokens (hybrid large-M regime: hot experts on the wide kernel, cold
+    """A small layer at 600 tokens (hybrid large-M regime: hot experts on the prefill kernel, cold
     ones on the small kernel, here on one stream) then 40 tokens."""
     spec = synth.scaled_spec("c1", hidden_size=512, num_experts=16, moe_intermediate_size=256,
                              shared_expert_intermediate_size=256)
