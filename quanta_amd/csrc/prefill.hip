@@ -273,12 +273,10 @@ __global__ void __launch_bounds__(kPfThreads, 1) prefill_kernel(QmmArgs a) {
     for (int nb = 0; nb < NB; ++nb) rex[nb] = rl.ex[nb] - DS;
     if (a_on && (lane & 3) == 0) row_tab[arow_r] = (arow >= 0) ? rl.rs : -1.0f;
   }
-  // scale/bias and high-bit copies: lanes 0-31 take an n-block's first tile, lanes 32-63 its second, the next one
-  // (32-bit offsets), or SwiGLU's up tile half the expert away (64-bit addresses)
-  constexpr bool FAR = EPI == EPI_SWIGLU && NB == 1;
-  const uint32_t sb_voff = 4 * r32 + hh * 128 * nsb, hb_voff = 16 * r32 + hh * C::SBB * nsb;
-  const char* sb_far = FAR ? wsb[hh ? 1 : 0] + 4 * r32 : nullptr;
-  const char* hb_far = FAR ? wtile[hh ? 1 : 0] + 1024 + 16 * r32 : nullptr;
+  // scale/bias and high-bit copies: lanes 0-31 take an n-block's first tile, lanes 32-63 its second
+  const int64_t t_step = static_cast<int64_t>(tile_of(1) - tile_of(0)) * nsb;
+  const uint32_t sb_voff = static_cast<uint32_t>(hh * t_step * 128 + 4 * r32);
+  const uint32_t hb_voff = static_cast<uint32_t>(hh * t_step * C::SBB + 16 * r32);
 
   // load u of superblock p into the slot at byte `slot`: the weights' C::LOADS, then A's 4 (when a_on)
   auto issue = [&](int p, int slot, int u, auto mbc) __attribute__((always_inline)) {
@@ -293,13 +291,10 @@ __global__ void __launch_bounds__(kPfThreads, 1) prefill_kernel(QmmArgs a) {
         dma16s(wtile[u] + static_cast<int64_t>(p) * C::SBB, 16 * lane, dst + u * C::CB);
     } else if (u < NC + NB) {
       const int nb = u - NC;
-      if (FAR) dma4(sb_far + static_cast<int64_t>(p) * 128, dst + C::NT * C::CB);
-      else dma4s(wsb[2 * nb] + static_cast<int64_t>(p) * 128, sb_voff, dst + C::NT * C::CB + 256 * nb);
+      dma4s(wsb[2 * nb] + static_cast<int64_t>(p) * 128, sb_voff, dst + C::NT * C::CB + 256 * nb);
     } else if (u < C::LOADS) {
       const int nb = u - NC - NB;
-      const uint32_t hd = dst + C::NT * (C::CB + 128) + 1024 * nb;
-      if (FAR) dma16(hb_far + static_cast<int64_t>(p) * C::SBB, hd);
-      else dma16s(wtile[2 * nb] + static_cast<int64_t>(p) * C::SBB + 1024, hb_voff, hd);
+      dma16s(wtile[2 * nb] + static_cast<int64_t>(p) * C::SBB + 1024, hb_voff, dst + C::NT * (C::CB + 128) + 1024 * nb);
     } else if (a_on) {
       const int q = u - C::LOADS;
       dma16(arow_ptr + 256 * p + 64 * q, lds_base + slot + (4 * wave + q) * 1024);

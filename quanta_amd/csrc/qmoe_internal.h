@@ -443,8 +443,7 @@ constexpr int kLargeMTile = 128;
 //                               789 / 810, 12.5 833 / 807, 14 913 / 830; c2 int6 10.5 1186 / 1197, 14 1411 / 1236;
 //                               512 experts 2048 x 512 11 261 / 270, 12 272 / 271; 128 of 4096 x 2048 int4 12 419 /
 //                               439, 14 459 / 431, int6 11 612 / 626, 12 647 / 638
-// (Skewed tokens, whose cold experts are smaller, still gain above the limit: c2 700 702 / 729. The host does not
-// know the skew.) The second tile's weights must still come from L2: above 8 M weights per projection they are read from
+// The second tile's weights must still come from L2: above 8 M weights per projection they are read from
 // HBM again (c3 376 tokens 1428 / 1345, c3 352 int6 2136 / 1979).
 constexpr int kHybridSplitRows = 16;
 inline bool few_hot(int64_t mc, int64_t n_experts, int64_t inter, int64_t hidden, int bits) {
