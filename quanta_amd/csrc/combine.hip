@@ -521,6 +521,11 @@ static bool fp16_large_fmt_q(int qfmt) {
   return qfmt == QMOE_FMT_INT4_G64 || qfmt == QMOE_FMT_INT6_G64 || qfmt == QMOE_FMT_INT3_G64;
 }
 
+// (AWQ runs gate and up without the SwiGLU epilogue; mixed widths by stacks of their own formats)
+static bool gate_up_reach(const qmoe_config_t& c) {
+  return c.awq || c.mixed || prefill_reach(kernel_fmt(c.expert_format), 2 * static_cast<int64_t>(c.inter), c.hidden);
+}
+
 static bool has_split(const qmoe_mixed_t& m) {
   for (int i = 0; i < m.n_stacks; ++i)
     if (m.stacks[i].proj == QMOE_PROJ_GATE || m.stacks[i].proj == QMOE_PROJ_UP) return true;
@@ -570,6 +575,8 @@ static int validate_config(const qmoe_config_t& c) {
   if (c.awq && c.regime == QMOE_REGIME_LARGE && !awq_large_ok(c))
     return fail("config: awq scales in the large regime need inter % 256 == 0");
   if (c.mixed != 0 && c.mixed != 1) return fail("config: mixed must be 0 or 1");
+  if (c.regime == QMOE_REGIME_LARGE && !gate_up_reach(c))
+    return fail("config: gate and up tiles more than 4 GiB apart need the small regime");
   if (c.mixed && c.awq) return fail("config: mixed-width experts run without awq scales");
   if (c.router_format == QMOE_ROUTER_BF16_TILED) {
     if (c.router_rows < c.n_experts + (c.shared_gated ? 1 : 0) || c.router_rows % 256)
@@ -688,6 +695,7 @@ extern "C" int qmoe_set_route_tail(int on) {
 static int pick_regime(const qmoe_config_t& c, int64_t N) {
   if (c.regime != QMOE_REGIME_AUTO) return c.regime;
   if (c.awq && !awq_large_ok(c)) return QMOE_REGIME_SMALL;
+  if (!gate_up_reach(c)) return QMOE_REGIME_SMALL;
   return large_ok(c, N) ? QMOE_REGIME_LARGE : QMOE_REGIME_SMALL;
 }
 

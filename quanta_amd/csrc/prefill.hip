@@ -24,7 +24,7 @@ constexpr int kPfABytes = 128 * 128 * 2;           // one superblock of 128 rows
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
   return __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p)));
 }
-// Global -> LDS copy: each lane's 16 (or 4) bytes at src land at lds_off + 16 (or 4) * lane.
+// Global -> LDS copy: each lane's 16 bytes at src land at lds_off + 16 * lane.
 // M0 is saved and restored around the copy.
 __device__ __forceinline__ void dma16(const void* src, uint32_t lds_off) {
   uint32_t saved;
@@ -32,14 +32,8 @@ __device__ __forceinline__ void dma16(const void* src, uint32_t lds_off) {
                "global_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
                : "=&s"(saved) : "v"(src), "s"(lds_off) : "memory");
 }
-__device__ __forceinline__ void dma4(const void* src, uint32_t lds_off) {
-  uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
-               "global_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "v"(src), "s"(lds_off) : "memory");
-}
-// The same copies from a wave-uniform base address (a scalar register pair) plus a 32-bit
-// per-lane offset: the base costs no vector registers.
+// The same copy, and one of 4 bytes per lane, from a wave-uniform base address (a scalar register pair) plus a
+// 32-bit per-lane offset: the base costs no vector registers.
 __device__ __forceinline__ void dma16s(const void* sbase, uint32_t voff, uint32_t lds_off) {
   uint32_t saved;
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
@@ -761,6 +755,8 @@ static int launch_prefill(const QmmArgs& a, int64_t mtiles, hipStream_t stream) 
 }
 
 int launch_large(const QmmArgs& a, int fmt, int epi, int64_t mtiles, hipStream_t stream) {
+  if (epi == EPI_SWIGLU && !prefill_reach(fmt, a.n_rows, a.K))
+    return fail("qmm(large): gate and up tiles more than 4 GiB apart (the small regime takes them)");
 #define QMOE_LARGE(F)                                                                  \
   (epi == EPI_SWIGLU ? launch_prefill<F, EPI_SWIGLU>(a, mtiles, stream)                \
    : epi == EPI_BF16 ? launch_prefill<F, EPI_BF16>(a, mtiles, stream)                  \

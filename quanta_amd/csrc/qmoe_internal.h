@@ -317,6 +317,14 @@ int launch_qmm(const QmmArgs& a, int fmt, int epi, int regime, int64_t mtile_bou
 int launch_dense(const QmmArgs& a, int fmt, int epi, hipStream_t stream);   // (dense.hip)
 // The large regime's launches (prefill.hip); launch_qmm has checked the arguments.
 int launch_large(const QmmArgs& a, int fmt, int epi, int64_t mtiles, hipStream_t stream);
+// Whether the prefill kernel reaches a SwiGLU stack's up tiles: with 256-row blocks their scales and high bits
+// are copied at 32-bit byte offsets from the gate tiles' (64-bit addresses cost int6 layers 1 %: c2 1000 tokens
+// 1313 / 1327 us). Short of it: 1.1e10 int6, 1.7e10 int4 or 2.3e10 int3 weights in one expert's gate_up.
+inline bool prefill_reach(int fmt, int64_t n_rows, int64_t K) {
+  if (!fmt_quant(fmt) || (fmt != FMT_INT6 && n_rows % 512 == 0)) return true;
+  const int64_t sb = fmt == FMT_INT6 ? 1536 : fmt == FMT_INT3 ? 768 : 1024;
+  return n_rows / 32 * (K / 128) * sb <= 0xffffffffll - 1024;
+}
 // Dense bf16 x bf16 -> fp32 (router logits), each sum in the large regime's order (prefill.hip).
 int launch_router_logits(const QmmArgs& a, hipStream_t stream);
 // Chunk count of the small-regime bf16 products over K: ~8 32-deep steps per chunk, one
@@ -443,7 +451,8 @@ constexpr int kLargeMTile = 128;
 //                               789 / 810, 12.5 833 / 807, 14 913 / 830; c2 int6 10.5 1186 / 1197, 14 1411 / 1236;
 //                               512 experts 2048 x 512 11 261 / 270, 12 272 / 271; 128 of 4096 x 2048 int4 12 419 /
 //                               439, 14 459 / 431, int6 11 612 / 626, 12 647 / 638
-// The second tile's weights must still come from L2: above 8 M weights per projection they are read from
+// (Skewed tokens, whose cold experts are smaller, still gain above the limit: c2 700 702 / 729. The host does not
+// know the skew.) The second tile's weights must still come from L2: above 8 M weights per projection they are read from
 // HBM again (c3 376 tokens 1428 / 1345, c3 352 int6 2136 / 1979).
 constexpr int kHybridSplitRows = 16;
 inline bool few_hot(int64_t mc, int64_t n_experts, int64_t inter, int64_t hidden, int bits) {

@@ -325,3 +325,19 @@ def test_router_one_call_validation(args, fragment):
                          a["scale"], a["idx"], a["w"], a["sg_out"], a["ws"], a["ws_bytes"], None)
     assert rc == L.QMOE_EINVAL and fragment in _last_error(), _last_error()
     assert lib.qmoe_router_workspace(4, 16) >= 4 * 17 * 4
+
+
+@pytest.mark.parametrize("fmt,inter,ok", [(2, 87296, True), (2, 87424, False), (0, 131072, True), (0, 131200, False),
+                                          (0, 131328, True), (3, 174720, True), (3, 174848, True), (3, 174976, False),
+                                          (1, 262144, True)])
+def test_forced_large_regime_reach(fmt, inter, ok):
+    """int6, and int3 and int4 in 256-row blocks: gate and up tiles of one expert at hidden 65536 on either side of
+    4 GiB apart; other formats and 512-row blocks have no such bound. (Beyond it the automatic regime is the
+    small one.)"""
+    cfg = L.QmoeConfig(hidden=65536, n_experts=2, top_k=1, inter=inter, shared_inter=0, scoring=0, norm_topk=1,
+                       n_group=1, topk_group=1, routed_scale=1.0, expert_format=fmt, down_format=fmt,
+                       router_format=1, router_rows=0, shared_gated=0, regime=2)
+    dummy = ctypes.c_void_p(16)
+    rc = L.load().qmoe_forward(ctypes.byref(cfg), ctypes.byref(L.QmoeWeights()), dummy, 300, dummy, dummy, 16, None)
+    assert rc == L.QMOE_EINVAL
+    assert ("4 GiB apart" not in _last_error()) == ok   # (the next check, the workspace's size, refuses the others)
